@@ -293,7 +293,7 @@ int qq_init(int device, qq_ctx **out)
     }
     void *sync = nullptr;
     const size_t sync_bytes = sync_table_words() * sizeof(uint64_t) + 512 + SEG_CTR_WORDS * 4 + 256 +
-                              (size_t)ctx->num_cus * SEG_PART_WORDS * 8;
+                              (size_t)ctx->num_cus * (SEG_PART_WORDS * 8 + 32768);
     if ((e = hipMalloc(&sync, sync_bytes)) != hipSuccess || (e = hipMemset(sync, 0, sync_bytes)) != hipSuccess) {
         if (sync) (void)hipFree(sync);
         (void)hipEventDestroy(ctx->ev0);
@@ -316,6 +316,7 @@ int qq_init(int device, qq_ctx **out)
     ctx->sync_epoch = ctx->sync_err + 32;
     ctx->sync_seg = ctx->sync_err + 128;
     ctx->seg_part = reinterpret_cast<uint64_t *>(((uintptr_t)(ctx->sync_seg + SEG_CTR_WORDS) + 255) & ~(uintptr_t)255);
+    ctx->rows_part = reinterpret_cast<float *>(ctx->seg_part + (size_t)ctx->num_cus * SEG_PART_WORDS);
     ctx->capturing = 0;
     *out = ctx;
     return QQ_OK;

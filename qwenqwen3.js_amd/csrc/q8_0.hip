@@ -54,91 +54,6 @@ int launch_repack_q8_0(qq_ctx *ctx, const uint8_t *gguf_dev, qq_tensor *t)
 }
 
 // ---------------------------------------------------------------------------
-// Matvec over R input vectors.  A workgroup (4 waves) owns 32 output rows; lane l of every wave
-// takes row l/2 and half l%2 of a block, wave w takes block columns
-// w, w+4, ...  The R input vectors sit in LDS (a window of up to MV_WIN
-// blocks at a time) together with the sum of every 16-value half block.
-// Per lane: 16 weights x R vectors per block; lanes pair up at the end and
-// the 4 waves are summed through LDS in a fixed order.
-// ---------------------------------------------------------------------------
-// MV_WIN = blocks of activations staged per pass: 32 KiB of LDS for R vectors.
-template <int R, int MV_WIN = 256 / R>
-__global__ __launch_bounds__(256) void q8_0_matvec_kernel(
-    const int8_t *__restrict__ qs, const __half *__restrict__ dsc, int mat, int rows, int nb,
-    int in_dim, const float *__restrict__ x, int ldx, float *__restrict__ y, int ldy, int nvec)
-{
-    __shared__ __align__(16) float xl[R][MV_WIN * QK];
-    __shared__ float xs[R][2 * MV_WIN];
-    __shared__ float red[4][R][32];
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int wave = threadIdx.x / WAVE;
-    const int v0 = blockIdx.y * R;
-    const int row = blockIdx.x * 32 + lane / 2;
-    const int h = lane & 1;
-    const bool row_ok = row < rows;
-
-    float acc[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) acc[r] = 0.0f;
-
-    for (int b0 = 0; b0 < nb; b0 += MV_WIN) {
-        const int nbw = min(MV_WIN, nb - b0);
-        __syncthreads();
-        for (int i = threadIdx.x; i < R * nbw * QK; i += 256) {
-            const int r = i / (nbw * QK), kk = i - r * nbw * QK;
-            const int k = b0 * QK + kk;
-            xl[r][kk] = (v0 + r < nvec && k < in_dim) ? x[(size_t)(v0 + r) * ldx + k] : 0.0f;
-        }
-        __syncthreads();
-        for (int i = threadIdx.x; i < R * 2 * nbw; i += 256) {
-            const int r = i / (2 * nbw), hb = i - r * 2 * nbw;
-            float s = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 16; j++) s += xl[r][hb * 16 + j];
-            xs[r][hb] = s;
-        }
-        __syncthreads();
-        // four blocks per wave in flight
-        for (int bb = wave; bb < nbw; bb += 16) {
-            int4 q[4];
-            float dd[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {   // branch-free: clamped address, zero scale
-                const int b = bb + 4 * u;
-                const size_t o = bm_index(mat, nb, b0 + min(b, nbw - 1), rows, min(row, rows - 1));
-                q[u] = *reinterpret_cast<const int4 *>(qs + o * QK + 16 * h);
-                dd[u] = __half2float(dsc[o]);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) dd[u] = (row_ok && bb + 4 * u < nbw) ? dd[u] : 0.0f;
-            // all loads above are issued before any of the arithmetic below
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int b = bb + 4 * u;
-                if (b < nbw) {
-#pragma unroll
-                    for (int r = 0; r < R; r++)
-                        acc[r] = fmaf(dot16_q8_lds(q[u], &xl[r][b * QK + 16 * h], xs[r][2 * b + h]),
-                                      dd[u], acc[r]);
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        acc[r] += __shfl_xor(acc[r], 1, WAVE);
-        if (h == 0) red[wave][r][lane / 2] = acc[r];
-    }
-    __syncthreads();
-    if (threadIdx.x < R * 32) {
-        const int r = threadIdx.x / 32, rr = threadIdx.x % 32;
-        const int orow = blockIdx.x * 32 + rr;
-        if (orow < rows && v0 + r < nvec)
-            y[(size_t)(v0 + r) * ldy + orow] = ((red[0][r][rr] + red[1][r][rr]) + red[2][r][rr]) + red[3][r][rr];
-    }
-}
-
 // Single input vector.  A workgroup owns RPW output rows and all of their
 // block columns; lane l of a wave takes half h = l & 1 of a block, row
 // (l >> 1) % RPW and block slot l / (2 RPW), so one 16-byte load per lane
@@ -267,23 +182,15 @@ int launch_q8_0_matvec(qq_ctx *ctx, const qq_tensor *t, int mat, const float *x,
                        float *y, int ldy, int rows)
 {
     if (rows <= 0) return QQ_OK;
-    const unsigned gx = (unsigned)((t->out_dim + 31) / 32);
+    // one vector whose activations fit in LDS (in_dim <= 12288); everything
+    // else takes the row kernels
+    if (rows > 1 || ((uintptr_t)x & 15) != 0 || t->nb > MV1_MAX_NB)
+        return launch_q8_0_rows(ctx, t, mat, x, ldx, y, ldy, rows);
     prof_begin(ctx, K_MATVEC);
-    // one vector whose activations fit in LDS (in_dim <= 12288)
-    if (rows == 1 && ((uintptr_t)x & 15) == 0 && t->nb <= MV1_MAX_NB) {
-        if (t->in_dim % QK)
-            launch_matvec1<true>(ctx, t, mat, x, y);
-        else
-            launch_matvec1<false>(ctx, t, mat, x, y);
-    } else if (rows >= 4)
-        QQ_LAUNCH(ctx, (q8_0_matvec_kernel<4>), dim3(gx, (rows + 3) / 4), dim3(256), 0, t->qs, t->d, mat, t->out_dim, t->nb, t->in_dim, x, ldx, y,
-                           ldy, rows);
-    else if (rows >= 2)
-        QQ_LAUNCH(ctx, (q8_0_matvec_kernel<2>), dim3(gx, (rows + 1) / 2), dim3(256), 0, t->qs, t->d, mat, t->out_dim, t->nb, t->in_dim, x, ldx, y,
-                           ldy, rows);
+    if (t->in_dim % QK)
+        launch_matvec1<true>(ctx, t, mat, x, y);
     else
-        QQ_LAUNCH(ctx, (q8_0_matvec_kernel<1>), dim3(gx, rows), dim3(256), 0,
-                           t->qs, t->d, mat, t->out_dim, t->nb, t->in_dim, x, ldx, y, ldy, rows);
+        launch_matvec1<false>(ctx, t, mat, x, y);
     prof_end(ctx);
     QQ_HIP(ctx, hipGetLastError());
     return QQ_OK;

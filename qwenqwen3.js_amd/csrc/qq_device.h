@@ -278,22 +278,6 @@ __device__ __forceinline__ float dot16_q8(const int4 q, const float *x, float xs
     return fmaf(-128.0f, xsum, acc);
 }
 
-// Same, activations read from LDS as four float4.
-__device__ __forceinline__ float dot16_q8_lds(const int4 q, const float *xl, float xsum)
-{
-    float xr[16];
-    const float4 *p = reinterpret_cast<const float4 *>(xl);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float4 v = p[i];
-        xr[4 * i] = v.x;
-        xr[4 * i + 1] = v.y;
-        xr[4 * i + 2] = v.z;
-        xr[4 * i + 3] = v.w;
-    }
-    return dot16_q8(q, xr, xsum);
-}
-
 // Hide a register value from loop-invariant code motion: without it the
 // compiler hoists the int8->float conversion of every weight out of a token
 // loop and runs out of registers.

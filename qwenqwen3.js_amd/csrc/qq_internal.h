@@ -159,6 +159,7 @@ struct qq_ctx {
     uint64_t *sync_hloc, *sync_hdev, *sync_part, *sync_arrive, *sync_hx, *sync_rp, *sync_ri;
     uint32_t *sync_seg;   // SEG_CTR_WORDS stream-kernel segment counters and generations
     uint64_t *seg_part;   // num_cus x SEG_PART_WORDS partial sums
+    float *rows_part;     // num_cus x 32 KiB: partial sums of split Q8_0 row products (rows.hip)
     // device-side waits that timed out on this context so far (counted when
     // the error word is read); device-resident state built across calls (an
     // LFM2 model's conv states and KV cache) is invalid after one
@@ -250,6 +251,9 @@ int launch_stage_copy(qq_ctx *ctx, const void *src, void *dst, size_t bytes);
 int launch_repack_q8_0(qq_ctx *ctx, const uint8_t *gguf_dev, qq_tensor *t);
 int launch_q8_0_matvec(qq_ctx *ctx, const qq_tensor *t, int mat, const float *x, int ldx,
                        float *y, int ldy, int rows);
+// ... its row kernels (rows.hip): any number of rows, any alignment
+int launch_q8_0_rows(qq_ctx *ctx, const qq_tensor *t, int mat, const float *x, int ldx, float *y, int ldy,
+                     int rows);
 // Router of a token batch: binary64 partial logits (router_work_bytes of
 // scratch at `part`), then top-K.
 constexpr int ROUTER_MAX_SPLIT = 8;

@@ -1,0 +1,116 @@
+"""Q8_0 matrix times several rows (rows.hip) against binary64 sums.
+
+Tolerance: activations enter exactly (three bf16 planes), so the error is that
+of fp32 sums: at most ~60 roundings of 2^-24 in a row (16 blocks a level, the
+levels, waves and segments), 3.6e-6 at worst and ~1e-7 as the roundings fall.
+"""
+import numpy as np
+import pytest
+
+import synth
+from _util import gpu_context, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-6
+
+
+def _dense(w, in_dim, out_dim):
+    b = np.asarray(w).view(synth.Q8_DTYPE).reshape(out_dim, -1)
+    m = b["qs"].astype(np.float64) * b["d"].astype(np.float64)[..., None]
+    return m.reshape(out_dim, -1)[:, :in_dim]
+
+
+def _case(in_dim, out_dim, rows, seed=0):
+    rng = np.random.default_rng([in_dim, out_dim, rows, seed])
+    w = synth.q8_0_tensor(rng, in_dim, out_dim)
+    x = rng.standard_normal((rows, in_dim)).astype(np.float32)
+    return w, x, x.astype(np.float64) @ _dense(w, in_dim, out_dim).T
+
+
+@pytest.mark.parametrize("in_dim,out_dim,rows", [
+    (2048, 200, 2), (2048, 200, 16),        # one 16-row tile, one column fragment
+    (2048, 4100, 5),                        # two column fragments, partial last group
+    (64, 32768, 3),                         # four column fragments
+    (2048, 200, 17), (2048, 200, 32),       # two row fragments, last row of the row kernel
+    (2048, 2100, 31),                       # two row x two column fragments
+    (64, 8200, 32),                         # two row x four column fragments
+    (1024, 70, 64),                         # rows x blocks at the GEMM's threshold ...
+    (1024, 70, 65),                         # ... and past it: partial second row tile
+    (2048, 31, 33), (7168, 129, 40),        # partial column groups, steps split over workgroups
+    (2048, 1, 200),                         # a single output
+    (96, 300, 700),                         # 3 blocks: an odd count, one segment
+    (2080, 777, 130),                       # 65 blocks, odd output count
+    (32, 40, 2100),                         # one block
+    (512, 16500, 200),                      # 256-output groups
+    (1000, 1501, 4), (1000, 1501, 20), (1000, 1501, 150),   # in_dim % 32 != 0, rows 16-byte aligned
+    (1001, 77, 9), (1003, 77, 40), (33, 300, 300),          # rows at any 4-byte alignment
+])
+def test_rows(in_dim, out_dim, rows):
+    print("rows", in_dim, out_dim, rows, flush=True)
+    w, x, ref = _case(in_dim, out_dim, rows)
+    t = gpu_context().upload_q8_0(w, in_dim, out_dim)
+    try:
+        y = t.matvec(x)
+    finally:
+        t.release()
+    assert np.isfinite(y).all()
+    for r in range(rows):
+        assert rel_l2(y[r], ref[r]) < TOL or out_dim == 1, (r, rel_l2(y[r], ref[r]))
+    assert rel_l2(y, ref) < TOL
+
+
+@pytest.mark.parametrize("in_dim,rows", [(512, 8), (512, 24), (2048, 80), (1000, 80)])
+def test_rows_special_values(in_dim, rows):
+    """Infinities, NaN and large or small rows stay with their own row; a
+    power of two on a row is a power of two on its result."""
+    out_dim = 96
+    w, x, ref = _case(in_dim, out_dim, rows, 1)
+    x[1] *= np.float32(2.0 ** 100)
+    x[2] *= np.float32(2.0 ** -80)
+    x[3, 7] = np.inf
+    x[4, in_dim - 1] = -np.inf
+    x[5, 40] = np.nan
+    x[6, 3] = np.array([0x7f800001], np.uint32).view(np.float32)[0]   # a NaN with only a low payload bit
+    t = gpu_context().upload_q8_0(w, in_dim, out_dim)
+    try:
+        y = t.matvec(x)
+    finally:
+        t.release()
+    q = np.asarray(w).view(synth.Q8_DTYPE).reshape(out_dim, -1)["qs"].reshape(out_dim, -1)
+    for r, k, s in ((3, 7, 1.0), (4, in_dim - 1, -1.0)):
+        want = np.where(q[:, k] == 0, np.nan, s * np.sign(q[:, k]) * np.inf)
+        np.testing.assert_array_equal(y[r], want.astype(np.float32))
+    assert np.isnan(y[5]).all() and np.isnan(y[6]).all()
+    ref[1] *= 2.0 ** 100
+    ref[2] *= 2.0 ** -80
+    for r in [0, 1, 2] + list(range(7, rows)):
+        assert rel_l2(y[r], ref[r]) < TOL, r
+
+
+def test_rows_captured():
+    """A recorded call needs nothing the context did not already hold, and
+    replays to the eager result."""
+    import torch
+    ctx = gpu_context()
+    in_dim, out_dim, rows = 2048, 512, 100
+    w, x, _ = _case(in_dim, out_dim, rows, 2)
+    t = ctx.upload_q8_0(w, in_dim, out_dim)
+    xd = torch.from_numpy(x).cuda()
+    y0, y1 = (torch.zeros((rows, out_dim), device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    ctx.capture_begin()
+    t.matvec_dev(xd.data_ptr(), y1.data_ptr(), rows)
+    g = ctx.capture_end()
+    try:
+        t.matvec_dev(xd.data_ptr(), y0.data_ptr(), rows)
+        ctx.synchronize()
+        for _ in range(3):
+            y1.zero_()
+            torch.cuda.synchronize()
+            g.launch()
+            ctx.synchronize()
+            assert torch.equal(y0, y1)
+    finally:
+        g.release()
+        t.release()
