@@ -81,6 +81,9 @@ __device__ __forceinline__ double rms_inv(double sumsq, int H, double eps)
 // Two int8 values of w (bytes LO, LO + 1) -> two fp16 halves holding the
 // same integers exactly: v_cvt_f16_i16 on a sign-extended byte (SDWA byte
 // select), the second written into the high half with the low half kept.
+// Inline assembly, so no wait states are kept between it and an MFMA in
+// flight: only for loops whose accumulators keep their registers (an output
+// placed where an MFMA still reads its addend corrupts that product).
 template <int LO>
 __device__ __forceinline__ uint32_t i8pair_f16(uint32_t w)
 {

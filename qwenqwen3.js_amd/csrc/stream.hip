@@ -4,8 +4,8 @@
 // With ~8 rows per expert (64 tokens, 32 experts, top-4) every weight is used
 // by very few rows, so the layer is bound by streaming the experts' Q8_0
 // weights from HBM once.  A workgroup owns one expert, one tile of 16*MF
-// slots and a group of weight columns (two halves of 16 NFH: 64 or 112 gate
-// and the same up features, 128 down columns); its 4 waves split the reduction
+// slots and a group of weight columns (two halves of 16 NFH: 32 to 112 gate
+// and the same up features, 64 to 128 down columns); its 4 waves split the reduction
 // dimension block by block (each streaming its blocks straight into
 // registers, a few blocks ahead, below) and their partial sums are added in
 // wave order through LDS.
@@ -21,6 +21,12 @@
 //            64 up columns; epilogue silu(g) * u -> act[slot][F] (fp32)
 //   down     A = act rows, B = 128 down columns -> y[slot][H] (fp32)
 // followed by the gather combine.
+//
+// us per call before / now, LFM2 shape (H 2048, F 1792, 32 experts, top-4):
+// 2 tokens 47 / 38, 6 tokens 71 / 56, 12 tokens 77 / 71, 64 tokens 86 / 83,
+// 128 tokens 120 / 113; Qwen3 shape (F 768, 128 experts, top-8): 16 tokens
+// 105 / 96, 64 tokens 139 / 130.  From the steady loop's unconditional loads
+// (st_mainloop) and, up to ~12 tokens, the width of the items (st_width).
 #include "qq_device.h"
 
 namespace qq {
@@ -69,13 +75,24 @@ __device__ __forceinline__ void split8(const float4 a, const float4 b, h8_t &hi,
 }
 
 // 8 int8 weights (one lane's share of a 16x32 fragment) -> 8 fp16 holding
-// the same integers exactly (four conversions per four weights; the
-// offset-binary form, bytes paired with the exponent byte 0x64 and 1152
-// subtracted, took five).
+// the same integers exactly: bytes in offset binary (q + 128) paired with the
+// exponent byte 0x64 give 1152 + q, and the subtraction is exact.  No inline
+// assembly here: the outputs may take the registers of a partial sum that an
+// MFMA in flight still reads, and the compiler keeps the wait states that
+// needs only between instructions it knows.
 __device__ __forceinline__ h8_t int8_to_f16x8(const uint2 q)
 {
-    return __builtin_bit_cast(h8_t, make_uint4(i8pair_f16<0>(q.x), i8pair_f16<2>(q.x), i8pair_f16<0>(q.y),
-                                               i8pair_f16<2>(q.y)));
+    const h2_t off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint32_t u = (i ? q.y : q.x) ^ 0x80808080u;
+        o[2 * i] = __builtin_bit_cast(
+            uint32_t, __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) + off);
+        o[2 * i + 1] = __builtin_bit_cast(
+            uint32_t, __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) + off);
+    }
+    return __builtin_bit_cast(h8_t, make_uint4(o[0], o[1], o[2], o[3]));
 }
 
 // ---------------------------------------------------------------------------
@@ -85,8 +102,8 @@ __device__ __forceinline__ h8_t int8_to_f16x8(const uint2 q)
 // bytes of each of the 2 NFH fragment columns (uint2) and one fp16 scale per
 // 64 columns of a half: load u of lane l reads column c0[h] + 64u + l's, and
 // a fragment's scale is taken from the lane that loaded it (fragment f of a
-// half: load f/4, lanes 16(f%4) .. 16(f%4)+15).  Each wave keeps st_pf
-// blocks in flight: block i + st_pf is requested as soon as block i's
+// half: load f/4, lanes 16(f%4) .. 16(f%4)+15).  Each wave keeps ST_PF
+// blocks in flight: block i + ST_PF is requested as soon as block i's
 // products are done.  (Staged through LDS the stream is held to ~100 KB in
 // flight per CU by the LDS size.)
 // Fragment j: column 16*(j%NFH) + lane%16 of half j/NFH; lane l holds row
@@ -101,9 +118,10 @@ struct StBlock {
     uint32_t ds[2][NS];  // scale bits of column c0[h] + 64 s + lane of half h
 };
 
-// blocks in flight per wave: ~12-14 KB of weights either way
-template <int MF, int NFH>
-constexpr int st_pf() { return MF == 1 && NFH == 4 ? 3 : 2; }
+// Blocks in flight per wave.  Two, at every width: 3 of the narrower ones took
+// longer (down at 64 tokens 26.3 us against 23.9, gate/up at 6 tokens 25.5
+// against 24.8).
+constexpr int ST_PF = 2;
 
 template <int MF, int NFH>
 struct StSrc {
@@ -182,31 +200,41 @@ __device__ __forceinline__ void st_block(const StBlock<MF, NFH> &b, const StSrc<
 }
 
 // Wave w reduces blocks kb0 + w, kb0 + w + 4, ... of the nb blocks from kb0
-// on, with st_pf blocks in flight.
+// on, with ST_PF blocks in flight.
 template <int MF, int NFH>
 __device__ __forceinline__ void st_mainloop(const StSrc<MF, NFH> &s, int kb0, int nb, int wave,
                                             f4_t (&acc)[MF][2 * NFH])
 {
-    constexpr int PF = st_pf<MF, NFH>();
+    constexpr int PF = ST_PF;
     const int nblk = (nb - wave + 3) / 4;
     const int kw = kb0 + wave;
     StBlock<MF, NFH> r[PF];
+    // Every load of the steady loop is unconditional: a wait for one block
+    // then leaves the blocks behind it in flight.  (Past a branch that may or
+    // may not have issued loads the compiler has to wait for all of them: so
+    // it drained every block in flight once per PF blocks.)
 #pragma unroll
-    for (int u = 0; u < PF; u++)
-        if (u < nblk) st_load<MF, NFH>(r[u], s, kw + 4 * u);
-    for (int i = 0; i < nblk; i += PF) {
+    for (int u = 0; u < PF; u++) st_load<MF, NFH>(r[u], s, min(kw + 4 * u, kb0 + nb - 1));
+    int i = 0;
+    for (; i + 2 * PF <= nblk; i += PF) {
 #pragma unroll
         for (int u = 0; u < PF; u++) {
-            if (i + u < nblk) {
-                st_block<MF, NFH>(r[u], s, acc);
-                // the refill goes out only after the products, so the
-                // compiler waits for this block alone, not the ones behind it
-                __builtin_amdgcn_sched_barrier(0);
-                if (i + u + PF < nblk) st_load<MF, NFH>(r[u], s, kw + 4 * (i + u + PF));
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            st_block<MF, NFH>(r[u], s, acc);
+            // the refill goes out only after the products
+            __builtin_amdgcn_sched_barrier(0);
+            st_load<MF, NFH>(r[u], s, kw + 4 * (i + u + PF));
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
+#pragma unroll
+    for (int u = 0; u < PF; u++)
+        if (i + u < nblk) {
+            st_block<MF, NFH>(r[u], s, acc);
+            if (i + u + PF < nblk) st_load<MF, NFH>(r[u], s, kw + 4 * (i + u + PF));
+        }
+#pragma unroll
+    for (int u = 0; u < PF; u++)
+        if (i + u + PF < nblk) st_block<MF, NFH>(r[u], s, acc);
 }
 
 // Load offsets: activation row r of the tile has byte offset rowoff(r);
@@ -273,6 +301,25 @@ constexpr int st_lds() { return 2 * 4 * 16 * (16 * NFH + 1) * 4; }
 // release / acquire pair, whose device-scope fences would write back the
 // whole L2.
 constexpr int ST_SEG_MAX = 8;   // segments of a split item
+
+// Width (NFH: fragments of 16 columns a half) of a launch that few tokens make:
+// the narrowest from LO to HI at which n row tiles are one round of the G
+// resident workgroups.  Each workgroup streams at a rate set by its own blocks
+// in flight, so with few tiles the time is that of one item, and an item's
+// time is its width (gate/up, one round: 15 us at 2, 24.8 at 4, 43.7 at 7).
+// The count of row tiles is known on the device only (the experts a few tokens
+// touch), so every workgroup works the width out; the sums do not depend on it.
+constexpr int ST_GU_MIN = 2, ST_GU_MAX = 7, ST_DN_MIN = 2, ST_DN_MAX = 4;
+
+template <int LO, int HI>
+__host__ __device__ inline int st_width(int n, int cols, int G)
+{
+    int best = HI;
+#pragma unroll
+    for (int w = HI - 1; w >= LO; w--)
+        if (n * ((cols + 16 * w - 1) / (16 * w)) <= G) best = w;
+    return best;
+}
 
 struct StWork {
     int item;         // tile * ncg + column group
@@ -420,20 +467,19 @@ __device__ __forceinline__ float silu_mul(float g, float u)
 // same up features.
 // ---------------------------------------------------------------------------
 template <int MF, int NFH>
-__global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_gateup_kernel(StreamArgs a)
+__device__ __forceinline__ void st_gateup(const StreamArgs &a, int n_tiles, char *lds, int *sh_last)
 {
     constexpr int NC = 16 * NFH;   // features per workgroup
-    __shared__ __align__(16) char lds[st_lds<NFH>()];
-    __shared__ int sh_last;
     const int ncg = (a.F + NC - 1) / NC;
     StWork wk;
-    if (!st_work(min(*a.n_tiles, a.tile_cap) * ncg, a.G, a.nbH, ncg, 16 * MF, a.tile_m0, wk)) return;
+    if (!st_work(n_tiles * ncg, a.G, a.nbH, ncg, 16 * MF, a.tile_m0, wk)) return;
     const int tile = wk.item / ncg, cg = wk.item - tile * ncg;
     const int e = a.tile_e[tile], m0 = a.tile_m0[tile];
     const int n = min(16 * MF, a.counts[e] - m0);
     const int slot0 = a.offsets[e] + m0;
     const int f0 = cg * NC;
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
 
     StSrc<MF, NFH> src;
     src.abase = reinterpret_cast<const char *>(a.x);
@@ -484,7 +530,7 @@ __global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_gateup_kernel(Stream
             }
         }
     }
-    if (wk.nseg == 1 || !st_last(a.seg_ctr + wk.li, wk.nseg, &sh_last)) return;
+    if (wk.nseg == 1 || !st_last(a.seg_ctr + wk.li, wk.nseg, sh_last)) return;
     const uint64_t *p0 = a.part + (size_t)wk.li * wk.nseg * PSZ;
     constexpr int NC4 = NC / 4;
     for (int i = threadIdx.x; i < 16 * MF * NC4; i += ST_THREADS) {
@@ -501,24 +547,44 @@ __global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_gateup_kernel(Stream
     st_item_done(a.seg_gen, wk.L, tag);
 }
 
-// ---------------------------------------------------------------------------
-// down: 128 output columns h0 .. h0+127 (halves h0 and h0 + 64).
-// ---------------------------------------------------------------------------
-template <int MF>
-__global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_down_kernel(StreamArgs a)
+// NFH = 0: the width that the count of row tiles asks for (st_width).
+template <int MF, int NFH>
+__global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_gateup_kernel(StreamArgs a)
 {
-    constexpr int NFH = 4;
-    __shared__ __align__(16) char lds[st_lds<NFH>()];
+    __shared__ __align__(16) char lds[st_lds<NFH ? NFH : ST_GU_MAX>()];
     __shared__ int sh_last;
-    const int ncg = (a.H + 127) / 128;
+    const int n = min(*a.n_tiles, a.tile_cap);
+    if constexpr (NFH == 0) {
+        switch (st_width<ST_GU_MIN, ST_GU_MAX>(n, a.F, a.G)) {
+        case 2: st_gateup<1, 2>(a, n, lds, &sh_last); break;
+        case 3: st_gateup<1, 3>(a, n, lds, &sh_last); break;
+        case 4: st_gateup<1, 4>(a, n, lds, &sh_last); break;
+        case 5: st_gateup<1, 5>(a, n, lds, &sh_last); break;
+        case 6: st_gateup<1, 6>(a, n, lds, &sh_last); break;
+        default: st_gateup<1, 7>(a, n, lds, &sh_last); break;
+        }
+    } else {
+        st_gateup<MF, NFH>(a, n, lds, &sh_last);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// down: 32 NFH output columns from h0 on (halves h0 and h0 + 16 NFH).
+// ---------------------------------------------------------------------------
+template <int MF, int NFH>
+__device__ __forceinline__ void st_down(const StreamArgs &a, int n_tiles, char *lds, int *sh_last)
+{
+    constexpr int NH = 16 * NFH, NC = 2 * NH;   // columns of a half, of the item
+    const int ncg = (a.H + NC - 1) / NC;
     StWork wk;
-    if (!st_work(min(*a.n_tiles, a.tile_cap) * ncg, a.G, a.nbF, ncg, 16 * MF, a.tile_m0, wk)) return;
+    if (!st_work(n_tiles * ncg, a.G, a.nbF, ncg, 16 * MF, a.tile_m0, wk)) return;
     const int tile = wk.item / ncg, cg = wk.item - tile * ncg;
     const int e = a.tile_e[tile], m0 = a.tile_m0[tile];
     const int n = min(16 * MF, a.counts[e] - m0);
     const int slot0 = a.offsets[e] + m0;
-    const int h0 = cg * 128;
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const int h0 = cg * NC;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
 
     StSrc<MF, NFH> src;
     src.abase = reinterpret_cast<const char *>(a.act);
@@ -527,7 +593,7 @@ __global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_down_kernel(StreamAr
     src.db[0] = src.db[1] = a.dd + eb;
     src.qstep = (uint32_t)a.H * QK;
     src.dstep = (uint32_t)a.H;
-    const int c0[2] = {h0, h0 + 64};
+    const int c0[2] = {h0, h0 + NH};
     st_offsets<MF, NFH>(src, [&](int r) { return (uint32_t)(slot0 + min(r, n - 1)) * a.F * 4; }, c0,
                         a.H, lane);
 
@@ -542,10 +608,10 @@ __global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_down_kernel(StreamAr
     const uint32_t tag =
         wk.nseg > 1 ? __hip_atomic_load(a.seg_gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u : 0u;
     st_mainloop<MF, NFH>(src, kb0, kb1 - kb0, wave, acc);
-    float (*red0)[16][65] = reinterpret_cast<float (*)[16][65]>(lds);
-    float (*red1)[16][65] = red0 + 4;
-    // split item: partial [16 MF rows][128 columns] of each segment
-    constexpr int PSZ = 16 * MF * 128;
+    float (*red0)[16][NH + 1] = reinterpret_cast<float (*)[16][NH + 1]>(lds);
+    float (*red1)[16][NH + 1] = red0 + 4;
+    // split item: partial [16 MF rows][NC columns] of each segment
+    constexpr int PSZ = 16 * MF * NC;
     uint64_t *pp = a.part + (size_t)(wk.li * wk.nseg + wk.seg) * PSZ;
 #pragma unroll
     for (int m = 0; m < MF; m++) {
@@ -554,22 +620,22 @@ __global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_down_kernel(StreamAr
         __syncthreads();
         // the tile's rows only (a split item's last segment reads those alone)
         const int nr = min(16, n - 16 * m);
-        for (int i = threadIdx.x; i < nr * 128; i += ST_THREADS) {
-            const int row = i >> 7, c = i & 127;
+        for (int i = threadIdx.x; i < nr * NC; i += ST_THREADS) {
+            const int row = i / NC, c = i % NC;
             const int h = h0 + c;
-            const float v = wave_order_sum<NFH>(c < 64 ? red0 : red1, row, c & 63);
+            const float v = wave_order_sum<NFH>(c < NH ? red0 : red1, row, c < NH ? c : c - NH);
             if (wk.nseg > 1)
-                store_tagged(pp + (16 * m + row) * 128 + c, tag, __float_as_uint(v));
+                store_tagged(pp + (16 * m + row) * NC + c, tag, __float_as_uint(v));
             else if (h < a.H)
                 a.y[(size_t)(slot0 + 16 * m + row) * a.H + h] = v;
         }
     }
-    if (wk.nseg == 1 || !st_last(a.seg_ctr + wk.li, wk.nseg, &sh_last)) return;
+    if (wk.nseg == 1 || !st_last(a.seg_ctr + wk.li, wk.nseg, sh_last)) return;
     const uint64_t *p0 = a.part + (size_t)wk.li * wk.nseg * PSZ;
-    for (int i = threadIdx.x; i < 16 * MF * 32; i += ST_THREADS) {
-        const int row = i >> 5, c = 4 * (i & 31);
+    for (int i = threadIdx.x; i < 16 * MF * (NC / 4); i += ST_THREADS) {
+        const int row = i / (NC / 4), c = 4 * (i % (NC / 4));
         if (row >= n) continue;
-        const int o[1] = {row * 128 + c};
+        const int o[1] = {row * NC + c};
         float v[1][4];
         if (!st_seg_sum<PSZ, 1>(p0, o, wk.nseg, tag, a.wait_ticks, v)) atomicOr(a.err, 8u);
         float *dst = a.y + (size_t)(slot0 + row) * a.H + h0 + c;
@@ -578,6 +644,23 @@ __global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_down_kernel(StreamAr
             if (h0 + c + j < a.H) dst[j] = v[0][j];
     }
     st_item_done(a.seg_gen, wk.L, tag);
+}
+
+template <int MF, int NFH>
+__global__ __launch_bounds__(ST_THREADS, 2) void moe_stream_down_kernel(StreamArgs a)
+{
+    __shared__ __align__(16) char lds[st_lds<NFH ? NFH : ST_DN_MAX>()];
+    __shared__ int sh_last;
+    const int n = min(*a.n_tiles, a.tile_cap);
+    if constexpr (NFH == 0) {
+        switch (st_width<ST_DN_MIN, ST_DN_MAX>(n, a.H / 2, a.G)) {
+        case 2: st_down<1, 2>(a, n, lds, &sh_last); break;
+        case 3: st_down<1, 3>(a, n, lds, &sh_last); break;
+        default: st_down<1, 4>(a, n, lds, &sh_last); break;
+        }
+    } else {
+        st_down<MF, NFH>(a, n, lds, &sh_last);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -640,6 +723,29 @@ static int stream_gateup_nfh(const qq_ctx *ctx, const qq_moe *m, int T)
     return (int)best;
 }
 
+// Whether so few experts are expected to be touched that items of `ncg` column
+// groups a row tile leave a sixth or more of the resident workgroups without
+// one: the launch then takes its width from the tile count (the widths in one
+// kernel cost a full launch about 1.5 us: 83.0 -> 85 us at 64 tokens).
+static bool stream_few(const qq_ctx *ctx, const qq_moe *m, int T, int ncg)
+{
+    const double touched = m->E * (1.0 - pow(1.0 - (double)m->K / m->E, (double)T));
+    return stream_mf(m, T) == 1 && touched * ncg <= (2.0 * ctx->num_cus) * 5.0 / 6.0;
+}
+
+// Workgroups of a launch: 8 * ceil(items / 8) for the most items that a tile
+// count up to cap makes, at `ncg` column groups a tile or (few) at the width it takes.
+template <int LO, int HI>
+static unsigned stream_grid(bool few, int cap, int ncg, int cols, int G)
+{
+    int items = cap * ncg;
+    for (int n = 1; few && n <= cap; n++) {
+        const int w = st_width<LO, HI>(n, cols, G);
+        items = std::max(items, n * ((cols + 16 * w - 1) / (16 * w)));
+    }
+    return 8u * (unsigned)((items + 7) / 8);
+}
+
 int launch_moe_stream(qq_ctx *ctx, const qq_moe *m, const float *x, float *hidden, int T,
                       const MaskBits &mask, const int32_t *idx, const double *w, char *work,
                       bool dispatched)
@@ -689,31 +795,37 @@ int launch_moe_stream(qq_ctx *ctx, const qq_moe *m, const float *x, float *hidde
     a.G = 2 * ctx->num_cus;
     a.tile_cap = cap;
 
-    // a split item's partial sums: [16 MF rows][2 x 16 NFH or 128 columns]
-    if (16 * MF * std::max(2 * 16 * stream_gateup_nfh(ctx, m, T), 128) > SEG_PART_WORDS)
-        return set_error(ctx, "stream path: partial sums exceed %d words", SEG_PART_WORDS);
+    // a split item's partial sums: [16 MF rows][2 x 16 NFH columns]
+    static_assert(16 * 2 * 16 * ST_GU_MAX <= SEG_PART_WORDS && 16 * 2 * 16 * ST_DN_MAX <= SEG_PART_WORDS &&
+                  32 * 2 * 16 * 4 <= SEG_PART_WORDS, "partial sums of a segment");
 
-    // grids (st_work): 8 * ceil(items / 8) workgroups for the items of cap
-    // row tiles; split items' segments take the room past the items there are
+    // grids (st_work): 8 * ceil(items / 8) workgroups for the items of up to
+    // cap row tiles; split items' segments take the room past the items there are
     const int nfh = stream_gateup_nfh(ctx, m, T);
-    const unsigned g1 = 8u * (unsigned)(((size_t)cap * ((m->F + 16 * nfh - 1) / (16 * nfh)) + 7) / 8);
-    const unsigned g2 = 8u * (unsigned)(((size_t)cap * ((m->H + 127) / 128) + 7) / 8);
+    const int ncg1 = (m->F + 16 * nfh - 1) / (16 * nfh), ncg2 = (m->H + 127) / 128;
+    const bool few1 = stream_few(ctx, m, T, ncg1), few2 = stream_few(ctx, m, T, ncg2);
+    const dim3 g1(stream_grid<ST_GU_MIN, ST_GU_MAX>(few1, cap, ncg1, m->F, a.G));
+    const dim3 g2(stream_grid<ST_DN_MIN, ST_DN_MAX>(few2, cap, ncg2, m->H / 2, a.G));
     prof_begin(ctx, K_STREAM_GATEUP);
-    if (MF == 1 && nfh == 7)
-        QQ_LAUNCH(ctx, (moe_stream_gateup_kernel<1, 7>), dim3(g1), dim3(ST_THREADS), 0, a);
+    if (few1)
+        QQ_LAUNCH(ctx, (moe_stream_gateup_kernel<1, 0>), g1, dim3(ST_THREADS), 0, a);
+    else if (MF == 1 && nfh == 7)
+        QQ_LAUNCH(ctx, (moe_stream_gateup_kernel<1, 7>), g1, dim3(ST_THREADS), 0, a);
     else if (MF == 1)
-        QQ_LAUNCH(ctx, (moe_stream_gateup_kernel<1, 4>), dim3(g1), dim3(ST_THREADS), 0, a);
+        QQ_LAUNCH(ctx, (moe_stream_gateup_kernel<1, 4>), g1, dim3(ST_THREADS), 0, a);
     else
-        QQ_LAUNCH(ctx, (moe_stream_gateup_kernel<2, 4>), dim3(g1), dim3(ST_THREADS), 0, a);
+        QQ_LAUNCH(ctx, (moe_stream_gateup_kernel<2, 4>), g1, dim3(ST_THREADS), 0, a);
     prof_end(ctx);
     QQ_HIP(ctx, hipGetLastError());
     prof_begin(ctx, K_STREAM_DOWN);
     a.seg_ctr = ctx->sync_seg + SEG_CTR_WORDS / 2;
     a.seg_gen = ctx->sync_seg + 3 * SEG_CTR_WORDS / 4;
-    if (MF == 1)
-        QQ_LAUNCH(ctx, moe_stream_down_kernel<1>, dim3(g2), dim3(ST_THREADS), 0, a);
+    if (few2)
+        QQ_LAUNCH(ctx, (moe_stream_down_kernel<1, 0>), g2, dim3(ST_THREADS), 0, a);
+    else if (MF == 1)
+        QQ_LAUNCH(ctx, (moe_stream_down_kernel<1, 4>), g2, dim3(ST_THREADS), 0, a);
     else
-        QQ_LAUNCH(ctx, moe_stream_down_kernel<2>, dim3(g2), dim3(ST_THREADS), 0, a);
+        QQ_LAUNCH(ctx, (moe_stream_down_kernel<2, 4>), g2, dim3(ST_THREADS), 0, a);
     prof_end(ctx);
     QQ_HIP(ctx, hipGetLastError());
     return launch_combine(ctx, m, T, y, false, inv, w, hidden);
