@@ -656,8 +656,12 @@ static int forward_run(qq_ctx *ctx, const qq_moe *m, const float *x, float *hidd
             if ((rc = launch_moe_stream(ctx, m, cx, ch, tn, mask, ci, cw, work, true))) return rc;
             continue;
         }
+        // the rows' 1 / sqrt(mean square + eps) take the place of the x rows
+        // that the router forms itself
+        NormArgs na{};
+        if (nfused) na = NormArgs{norm->w, norm->eps, reinterpret_cast<double *>(xn + (size_t)t0 * m->H)};
         if ((rc = launch_router_topk(ctx, m, nfused ? ch : cx, tn, part, ci, cw, cp, xh, &xh_done,
-                                     nfused ? norm : nullptr)))
+                                     nfused ? &na : nullptr)))
             return rc;
         switch (path) {
         case PATH_MFMA: rc = launch_moe_mfma(ctx, m, cx, ch, tn, mask, ci, cw, work, xh_done); break;

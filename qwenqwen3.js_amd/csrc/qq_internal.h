@@ -284,6 +284,7 @@ bool stack_decode_supported(const qq_ctx *ctx, const qq_moe *m);
 struct NormArgs {
     const float *w;
     double eps;
+    double *inv = nullptr;   // T values of scratch (the router's norm only)
 };
 
 // The weights of one layer of the batch-1 decode kernel (a stack launch

@@ -55,6 +55,50 @@ struct RouterW {
 };
 
 // ---------------------------------------------------------------------------
+// inv[t] = 1 / sqrt(sum x^2 / H + eps) of row t, one wave per row, through
+// rmsnorm_kernel's binary64 tree: lane l plays threads 64 v + l of the
+// normalising block for v = 0 .. NORM_THREADS / 64 - 1.  Bound by reading the
+// rows once.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void row_inv_kernel(const float *__restrict__ x, int T, int H, double eps,
+                                                      double *__restrict__ inv)
+{
+    constexpr int NV = NORM_THREADS / WAVE;
+    constexpr int NJ = 4;   // values 4 x NORM_THREADS of the row per pass of loads
+    const int lane = threadIdx.x & (WAVE - 1), t = blockIdx.x * 4 + threadIdx.x / WAVE;
+    if (t >= T) return;
+    const float *hr = x + (size_t)t * H;
+    double s[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) s[v] = 0.0;
+    // thread 64 v + l adds k = 64 v + l + 512 j for j = 0, 1, ... in order;
+    // past H the term is an exact no-op (s + 0 with s >= +0)
+    for (int j0 = 0; j0 < H; j0 += NJ * NORM_THREADS) {
+        float q[NJ][NV];
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int v = 0; v < NV; v++) q[j][v] = hr[min(j0 + j * NORM_THREADS + WAVE * v + lane, H - 1)];
+        // every load above goes out before the first use
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int v = 0; v < NV; v++) asm volatile("" : "+v"(q[j][v]));
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int v = 0; v < NV; v++) {
+                const double d = j0 + j * NORM_THREADS + WAVE * v + lane < H ? (double)q[j][v] : 0.0;
+                s[v] = fma(d, d, s[v]);
+            }
+    }
+    double r = wave_sum_dpp(s[0]);
+#pragma unroll
+    for (int v = 1; v < NV; v++) r = r + wave_sum_dpp(s[v]);
+    if (lane == 0) inv[t] = rms_inv(r, H, eps);
+}
+
+// ---------------------------------------------------------------------------
 // Matrix-core logits.  Grid (ceil(T/16), KS, ceil(E/32)), 4 waves.  Lane l of
 // a wave loads 4 consecutive k of token row l%16 and of expert rows l%16 and
 // 16 + l%16 at k = k0 + 4*(l/16); the j-th of them feeds the j-th of four
@@ -63,90 +107,40 @@ struct RouterW {
 // accumulators are added in wave order.  part[ks][t][e] (binary64).
 // f64 accumulator layout: lane l, element r -> row 4r + l/16, column l%16.
 //
+// Rows past T and experts past E are loaded clamped and go into rows and
+// columns of the product that are not stored.
+//
 // NRM: x holds the residual rows, and the workgroup forms x = rmsnorm(row)
 // (src/lfm2-engine.js:251-252) itself as it loads them: out of nw (or unit
-// weights), eps and each token's 1 / sqrt(sum x^2 / H + eps), whose sum of
-// squares is rmsnorm_kernel's own binary64 tree (wave w takes tokens 4w ..
-// 4w + 3; lane l plays thread 64 v + l of the normalising block for v = 0 ..
-// NORM_THREADS / 64 - 1), so logits and fp16 rows equal those of the two
-// launches bit for bit.
+// weights) and inv[t] = 1 / sqrt(sum x^2 / H + eps) from row_inv_kernel, whose
+// sum of squares is rmsnorm_kernel's own binary64 tree, so logits and fp16
+// rows equal those of the two launches bit for bit.  (Every workgroup forming
+// the sums of its own 16 rows did so once per slice of H and expert group: 34
+// us at 700 tokens x 128 experts against 4.2 + 15.6, 34.5 at 4096 x 32 against
+// 7.1 + 21.7.)
 // ---------------------------------------------------------------------------
 template <bool Q8, bool NRM>
 __global__ __launch_bounds__(256) void router_mfma_kernel(const float *__restrict__ x, int T,
                                                           RouterW W, int kchunk,
                                                           double *__restrict__ part,
                                                           _Float16 *__restrict__ xh,
-                                                          const float *__restrict__ nw, double eps)
+                                                          const float *__restrict__ nw,
+                                                          const double *__restrict__ invp)
 {
     static_assert(!(Q8 && NRM), "the norm is formed on the F32 router path only");
     __shared__ double red[4][16][33];
-    __shared__ double sinv[16];
     const int t0 = blockIdx.x * 16, ks = blockIdx.y, e0 = blockIdx.z * 32;
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int r16 = lane & 15, kq = lane >> 4;
     const int t = t0 + r16;
-    const double tz = t < T ? 1.0 : 0.0;
     const float *xr = x + (size_t)min(t, T - 1) * W.H;
     const int ka = ks * kchunk, kb = min(W.H, ka + kchunk);
-    double inv = 1.0;
-    if constexpr (NRM) {
-        constexpr int NV = NORM_THREADS / WAVE;
-        constexpr int NJ = 4;   // values 4 x NORM_THREADS of a row per pass of loads
-        for (int i0 = 0; i0 < 4; i0 += 2) {
-            double s[2][NV];
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int v = 0; v < NV; v++) s[i][v] = 0.0;
-            // thread 64 v + l adds k = 64 v + l + 512 j for j = 0, 1, ... in
-            // order; past H the term is an exact no-op (s + 0 with s >= +0).
-            // Two tokens' loads of a pass go out together.
-            for (int j0 = 0; j0 < W.H; j0 += NJ * NORM_THREADS) {
-                float q[2][NJ][NV];
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    const float *hr = x + (size_t)min(t0 + 4 * wave + i0 + i, T - 1) * W.H;
-#pragma unroll
-                    for (int j = 0; j < NJ; j++)
-#pragma unroll
-                        for (int v = 0; v < NV; v++)
-                            q[i][j][v] = hr[min(j0 + j * NORM_THREADS + WAVE * v + lane, W.H - 1)];
-                }
-                // every load above goes out before the first use (a load under
-                // its own bounds branch is waited for inside that branch)
-#pragma unroll
-                for (int i = 0; i < 2; i++)
-#pragma unroll
-                    for (int j = 0; j < NJ; j++)
-#pragma unroll
-                        for (int v = 0; v < NV; v++) asm volatile("" : "+v"(q[i][j][v]));
-#pragma unroll
-                for (int i = 0; i < 2; i++)
-#pragma unroll
-                    for (int j = 0; j < NJ; j++)
-#pragma unroll
-                        for (int v = 0; v < NV; v++) {
-                            const int k = j0 + j * NORM_THREADS + WAVE * v + lane;
-                            const double d = k < W.H ? (double)q[i][j][v] : 0.0;
-                            s[i][v] = fma(d, d, s[i][v]);
-                        }
-            }
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                double r = wave_sum_dpp(s[i][0]);
-#pragma unroll
-                for (int v = 1; v < NV; v++) r = r + wave_sum_dpp(s[i][v]);
-                if (lane == 0) sinv[4 * wave + i0 + i] = rms_inv(r, W.H, eps);
-            }
-        }
-        __syncthreads();
-        inv = sinv[r16];
-    }
+    const double inv = NRM ? invp[min(t, T - 1)] : 1.0;
 
     d4_t acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
     auto step = [&](const float4 xv, const double (&wa)[4], const double (&wb)[4]) {
-        const double xd[4] = {(double)xv.x * tz, (double)xv.y * tz, (double)xv.z * tz,
-                              (double)xv.w * tz};
+        const double xd[4] = {(double)xv.x, (double)xv.y, (double)xv.z, (double)xv.w};
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(xd[j], wa[j], acc0, 0, 0, 0);
@@ -156,56 +150,66 @@ __global__ __launch_bounds__(256) void router_mfma_kernel(const float *__restric
     int k = ka + 16 * wave;
     if constexpr (!Q8) {
         // F32 router: the raw rows of RB steps are loaded before any of them
-        // is used (one round trip per RB steps, not per step); steps past
-        // the slice load clamped addresses and are skipped
-        constexpr int RB = 4;
+        // is used, and those of the next RB steps before the current ones are
+        // multiplied: two register sets, unconditional loads (with the norm, 4096
+        // tokens x 32 experts 25.4 us -> 21.7, 2048 x 128 42 -> 33).  Steps past
+        // the slice load clamped addresses and are skipped.
+        constexpr int RB = 2;
         const int ea = min(e0 + r16, W.E - 1), eb = min(e0 + 16 + r16, W.E - 1);
-        const double za = e0 + r16 < W.E ? 1.0 : 0.0, zb = e0 + 16 + r16 < W.E ? 1.0 : 0.0;
-        for (; k < kb; k += 64 * RB) {
-            float4 xv[RB], va[RB], vb[RB], nv[RB];
+        const float *wra = W.f32 + (size_t)ea * W.H, *wrb = W.f32 + (size_t)eb * W.H;
+        struct Set {
+            float4 x[RB], a[RB], b[RB], n[RB];
+        };
+        auto load = [&](Set &s, int k) {
 #pragma unroll
             for (int u = 0; u < RB; u++) {
                 const int kk = min(k + 64 * u, kb - 16) + 4 * kq;
-                xv[u] = *reinterpret_cast<const float4 *>(xr + kk);
-                va[u] = *reinterpret_cast<const float4 *>(W.f32 + (size_t)ea * W.H + kk);
-                vb[u] = *reinterpret_cast<const float4 *>(W.f32 + (size_t)eb * W.H + kk);
-                nv[u] = (NRM && nw) ? *reinterpret_cast<const float4 *>(nw + kk) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+                s.x[u] = *reinterpret_cast<const float4 *>(xr + kk);
+                s.a[u] = *reinterpret_cast<const float4 *>(wra + kk);
+                s.b[u] = *reinterpret_cast<const float4 *>(wrb + kk);
+                if constexpr (NRM) s.n[u] = *reinterpret_cast<const float4 *>((nw ? nw : xr) + kk);
             }
-            // keeps the loads above the skip test below (otherwise each is
-            // sunk into its step's branch and waited for there)
-#pragma unroll
-            for (int u = 0; u < RB; u++)
-                asm volatile("" : "+v"(xv[u].x), "+v"(xv[u].y), "+v"(xv[u].z), "+v"(xv[u].w),
-                                  "+v"(va[u].x), "+v"(va[u].y), "+v"(va[u].z), "+v"(va[u].w),
-                                  "+v"(vb[u].x), "+v"(vb[u].y), "+v"(vb[u].z), "+v"(vb[u].w));
-            if constexpr (NRM) {
-                // rmsnorm_kernel's out[k] = fp32(w[k] * x[k] * inv)
-#pragma unroll
-                for (int u = 0; u < RB; u++) {
-                    const float4 wv = nv[u];
-                    xv[u].x = (float)((double)wv.x * (double)xv[u].x * inv);
-                    xv[u].y = (float)((double)wv.y * (double)xv[u].y * inv);
-                    xv[u].z = (float)((double)wv.z * (double)xv[u].z * inv);
-                    xv[u].w = (float)((double)wv.w * (double)xv[u].w * inv);
-                }
-            }
+        };
+        auto mul = [&](Set &s, int k) {
 #pragma unroll
             for (int u = 0; u < RB; u++) {
                 if (k + 64 * u >= kb) break;
-                const double wa[4] = {(double)va[u].x * za, (double)va[u].y * za, (double)va[u].z * za,
-                                      (double)va[u].w * za};
-                const double wb[4] = {(double)vb[u].x * zb, (double)vb[u].y * zb, (double)vb[u].z * zb,
-                                      (double)vb[u].w * zb};
-                step(xv[u], wa, wb);
+                float4 xv = s.x[u];
+                if constexpr (NRM) {
+                    // rmsnorm_kernel's out[k] = fp32(w[k] * x[k] * inv)
+                    const float4 wv = nw ? s.n[u] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+                    xv.x = (float)((double)wv.x * (double)xv.x * inv);
+                    xv.y = (float)((double)wv.y * (double)xv.y * inv);
+                    xv.z = (float)((double)wv.z * (double)xv.z * inv);
+                    xv.w = (float)((double)wv.w * (double)xv.w * inv);
+                }
+                const double wa[4] = {(double)s.a[u].x, (double)s.a[u].y, (double)s.a[u].z, (double)s.a[u].w};
+                const double wb[4] = {(double)s.b[u].x, (double)s.b[u].y, (double)s.b[u].z, (double)s.b[u].w};
+                step(xv, wa, wb);
                 // the fp16 copy of x for the prefill GEMMs (xh != nullptr):
                 // every (token, k) of the slice once, rounded to nearest even
                 if (xh && t < T && blockIdx.z == 0) {
-                    const h2_t lo = {(_Float16)xv[u].x, (_Float16)xv[u].y};
-                    const h2_t hi = {(_Float16)xv[u].z, (_Float16)xv[u].w};
+                    const h2_t lo = {(_Float16)xv.x, (_Float16)xv.y};
+                    const h2_t hi = {(_Float16)xv.z, (_Float16)xv.w};
                     *reinterpret_cast<uint2 *>(xh + (size_t)t * W.H + k + 64 * u + 4 * kq) =
                         make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
                 }
             }
+        };
+        // (a wave past its slice loads clamped addresses and multiplies nothing)
+        Set s0, s1;
+        load(s0, k);
+        while (k < kb) {
+            load(s1, k + 64 * RB);
+            __builtin_amdgcn_sched_barrier(0);
+            mul(s0, k);
+            __builtin_amdgcn_sched_barrier(0);
+            k += 64 * RB;
+            load(s0, k + 64 * RB);
+            __builtin_amdgcn_sched_barrier(0);
+            mul(s1, k);
+            __builtin_amdgcn_sched_barrier(0);
+            k += 64 * RB;
         }
     } else {
         for (; k < kb; k += 64) {
@@ -678,7 +682,7 @@ int launch_router_topk(qq_ctx *ctx, const qq_moe *m, const float *x, int T, doub
 {
     if (xh_done) *xh_done = false;
     if (T <= 0) return QQ_OK;
-    if (norm && !(router_norm_supported(m, x, norm->w) && xh && xh_done))
+    if (norm && !(router_norm_supported(m, x, norm->w) && xh && xh_done && norm->inv))
         return set_error(ctx, "router: the norm is formed only by the F32 matrix-core router with fp16 rows");
     const bool q8 = m->router_type == QQ_TYPE_Q8_0;
     RouterW W;
@@ -690,20 +694,26 @@ int launch_router_topk(qq_ctx *ctx, const qq_moe *m, const float *x, int T, doub
     W.nb = (m->H + QK - 1) / QK;
     const int KS = ((uintptr_t)x & 15) == 0 ? router_split(m, T) : 1;
 
+    if (norm) {
+        prof_begin(ctx, K_RMSNORM);
+        QQ_LAUNCH(ctx, row_inv_kernel, dim3((T + 3) / 4), dim3(256), 0, x, T, m->H, norm->eps, norm->inv);
+        prof_end(ctx);
+        QQ_HIP(ctx, hipGetLastError());
+    }
     prof_begin(ctx, K_ROUTER_LOGITS);
     if (m->H % 16 == 0 && ((uintptr_t)x & 15) == 0) {
         const int kchunk = ((m->H + KS * 64 - 1) / (KS * 64)) * 64;
         const dim3 g((T + 15) / 16, KS, (m->E + 31) / 32);
         if (q8) {
             QQ_LAUNCH(ctx, (router_mfma_kernel<true, false>), g, dim3(256), 0, x, T, W, kchunk, part, nullptr,
-                      nullptr, 0.0);
+                      nullptr, nullptr);
         } else if (norm) {
             QQ_LAUNCH(ctx, (router_mfma_kernel<false, true>), g, dim3(256), 0, x, T, W, kchunk, part,
-                      static_cast<_Float16 *>(xh), norm->w, norm->eps);
+                      static_cast<_Float16 *>(xh), norm->w, norm->inv);
             *xh_done = true;
         } else {
             QQ_LAUNCH(ctx, (router_mfma_kernel<false, false>), g, dim3(256), 0, x, T, W, kchunk, part,
-                      static_cast<_Float16 *>(xh), nullptr, 0.0);
+                      static_cast<_Float16 *>(xh), nullptr, nullptr);
             if (xh && xh_done) *xh_done = true;
         }
     } else {
