@@ -105,6 +105,8 @@ def kernel_bytes(name, T, n_experts):
     if name in ("combine", "rmsnorm"):
         return 2 * T * H * 4
     if name == "q8_0_matvec":
+        if name in LFM2_BYTES:   # the output head of the LFM2 token
+            return LFM2_BYTES[name]
         return MV_OUT * (MV_IN // 32) * QBLK + MV_IN * 4 + MV_OUT * 4
     return LFM2_BYTES.get(name)
 
@@ -386,8 +388,9 @@ def run_lfm2(args, torch, ctx, stream):
     w_dense = 3 * Hh * info["n_ff"] * q8
     w_head = Hh * V * q8
     mv_bytes = n_conv * w_conv + n_attn * w_attn + ndense * w_dense + w_head
-    mv_launches = 2 * n_conv + 2 * n_attn + 2 * ndense + 1
-    LFM2_BYTES["lfm2_matvec"] = mv_bytes / mv_launches
+    mv_launches = 2 * n_conv + 2 * n_attn + 2 * ndense
+    LFM2_BYTES["lfm2_matvec"] = (mv_bytes - w_head) / mv_launches
+    LFM2_BYTES["q8_0_matvec"] = w_head + Hh * 4 + V * 4
     avg_n_prof = p0 + (n_prof + 1) / 2.0
     LFM2_BYTES["lfm2_attention"] = info["n_head_kv"] * avg_n_prof * 64 * 4 * 2
     LFM2_BYTES["lfm2_embed"] = Hh * q8 + Hh * 4
@@ -398,6 +401,7 @@ def run_lfm2(args, torch, ctx, stream):
     tok_bytes = mv_bytes + moe_bytes + kv_bytes
     kernels = kernel_table(prof, 1, K, K)
     dom, roofline = roofline_of(prof, kernels, args.workload)
+    del LFM2_BYTES["q8_0_matvec"]
     config = {"workload": "lfm2_8b_a1b_token_decode", "blocks": nl, "attention_blocks": n_attn,
               "dense_ffn_blocks": ndense, "moe_blocks": n_moe, "H": Hh, "heads": info["n_heads"],
               "kv_heads": info["n_head_kv"], "head_dim": info["head_dim"], "n_ff": info["n_ff"],

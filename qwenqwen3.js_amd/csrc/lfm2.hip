@@ -108,7 +108,7 @@ template <int MODE, int G, int RPW>
 __device__ __forceinline__ int lm_row(const LmArgs &a, int g, int &mat)
 {
     const int j = blockIdx.x;
-    if (MODE == LM_PLAIN || MODE == LM_RESID) {
+    if (MODE == LM_RESID) {
         mat = 0;
         return G * RPW * j + RPW * g;
     }
@@ -303,13 +303,13 @@ __global__ __launch_bounds__(G * WPG * WAVE) void lfm2_mv_kernel(LmArgs a)
         for (int w = 1; w < WPG; w++) v += red[gg][w][r];
         return v;
     };
-    if (MODE == LM_PLAIN || MODE == LM_RESID) {
+    if (MODE == LM_RESID) {
         if (tid < G * RPW) {
             const int gg = tid / RPW, r = tid % RPW;
             const int orow = G * RPW * blockIdx.x + RPW * gg + r;
             if (orow < a.m[0].rows) {
                 const float v = rowsum(gg, r);
-                a.y[orow] = MODE == LM_RESID ? yold + v : v;
+                a.y[orow] = yold + v;
             }
         }
     } else if (MODE == LM_SWIGLU) {
@@ -716,9 +716,6 @@ int launch_lfm2_mv(qq_ctx *ctx, int mode, const LmLaunch &l)
     // measured on the LFM2-8B-A1B token against 2 to 32 rows per group and 1
     // to 16 waves
     switch (mode) {
-    case LM_PLAIN:   // the output head: 65536 rows
-        mv_launch<LM_PLAIN, 1, 16, 4, 32>(ctx, (a.m[0].rows + 31) / 32, shm, a);
-        break;
     case LM_RESID:   // 2048 inputs (64 blocks), or the dense FFN's 7168 (224)
         if (a.nb <= 64)
             mv_launch<LM_RESID, 1, 8, 1, 4>(ctx, (a.m[0].rows + 3) / 4, shm, a);

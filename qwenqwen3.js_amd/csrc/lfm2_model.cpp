@@ -529,14 +529,8 @@ static int lfm2_forward(qq_ctx *ctx, qq_lfm2 *m, int token, int position, float 
     }
     if (logits_dev) {
         // output norm ("token_embd_norm.weight") and head
-        qq::LmLaunch o;
-        o.x = m->hidden;
-        o.mats[0] = m->output;
-        o.norm = 1;
-        o.norm_w = m->out_norm;
-        o.eps = I.eps;
-        o.y = logits_dev;
-        if (int rc = qq::launch_lfm2_mv(ctx, qq::LM_PLAIN, o)) return rc;
+        if (int rc = qq::launch_rmsnorm(ctx, m->hidden, m->out_norm, m->ybuf, 1, I.n_embd, I.eps)) return rc;
+        if (int rc = qq::launch_q8_0_matvec(ctx, m->output, 0, m->ybuf, I.n_embd, logits_dev, I.n_vocab, 1)) return rc;
     }
     return QQ_OK;
 }

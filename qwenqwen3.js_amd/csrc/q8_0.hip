@@ -67,6 +67,7 @@ int launch_repack_q8_0(qq_ctx *ctx, const uint8_t *gguf_dev, qq_tensor *t)
 // wave order.  RAG: in_dim is not a multiple of 32 (the missing activations
 // of the last block read as zero).
 constexpr int MV1_MAX_NB = 384;   // 48 KiB of activations in LDS
+constexpr int MV1_MAX_OUT = 16384;
 
 template <int RPW, int NWV, int NBW, bool RAG>
 __global__ __launch_bounds__(NWV * WAVE) void q8_0_matvec1_kernel(const int8_t *__restrict__ qs,
@@ -182,9 +183,11 @@ int launch_q8_0_matvec(qq_ctx *ctx, const qq_tensor *t, int mat, const float *x,
                        float *y, int ldy, int rows)
 {
     if (rows <= 0) return QQ_OK;
-    // one vector whose activations fit in LDS (in_dim <= 12288); everything
-    // else takes the row kernels
-    if (rows > 1 || ((uintptr_t)x & 15) != 0 || t->nb > MV1_MAX_NB)
+    // one vector whose activations fit in LDS (in_dim <= 12288), of a matrix of
+    // few enough outputs that staging them once per 8 outputs is cheap (us,
+    // this kernel / the row kernel, 2048 inputs: 7168 outputs 5.9 / 6.1, 16384
+    // 11.6 / 9.4, 65536 34.4 / 24.1); everything else takes the row kernels
+    if (rows > 1 || ((uintptr_t)x & 15) != 0 || t->nb > MV1_MAX_NB || t->out_dim >= MV1_MAX_OUT)
         return launch_q8_0_rows(ctx, t, mat, x, ldx, y, ldy, rows);
     prof_begin(ctx, K_MATVEC);
     if (t->in_dim % QK)

@@ -317,10 +317,10 @@ int launch_route_record(qq_ctx *ctx, const int32_t *idx, const double *w, const 
                         int K, int E, float *rec);
 size_t grouped_work_bytes(const qq_moe *m, int T);
 
-// LFM2 single-token forward (lfm2.hip).  Matvec modes: y = W x; hidden +=
+// LFM2 single-token forward (lfm2.hip).  Matvec modes: hidden +=
 // W x; silu(gate x) * (up x); in_proj + short-conv; raw q and k rows with v
 // stored into the KV cache.
-enum { LM_PLAIN = 0, LM_RESID = 1, LM_SWIGLU = 2, LM_CONV = 3, LM_QKV = 4 };
+enum { LM_RESID = 1, LM_SWIGLU = 2, LM_CONV = 3, LM_QKV = 4 };
 struct LmLaunch {
     const float *x = nullptr;
     const qq_tensor *mats[3] = {nullptr, nullptr, nullptr};

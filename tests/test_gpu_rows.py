@@ -44,6 +44,7 @@ def _case(in_dim, out_dim, rows, seed=0):
     (32, 40, 2100),                         # one block
     (512, 16500, 200),                      # 256-output groups
     (1000, 1501, 4), (1000, 1501, 20), (1000, 1501, 150),   # in_dim % 32 != 0, rows 16-byte aligned
+    (2048, 16383, 1), (2048, 16384, 1), (64, 40000, 1),     # one row: either side of the rule
     (1001, 77, 9), (1003, 77, 40), (33, 300, 300),          # rows at any 4-byte alignment
 ])
 def test_rows(in_dim, out_dim, rows):
@@ -79,7 +80,7 @@ def test_rows_special_values(in_dim, rows):
         t.release()
     q = np.asarray(w).view(synth.Q8_DTYPE).reshape(out_dim, -1)["qs"].reshape(out_dim, -1)
     for r, k, s in ((3, 7, 1.0), (4, in_dim - 1, -1.0)):
-        want = np.where(q[:, k] == 0, np.nan, s * np.sign(q[:, k]) * np.inf)
+        want = np.where(q[:, k] == 0, np.nan, np.where(q[:, k] > 0, s, -s) * np.inf)
         np.testing.assert_array_equal(y[r], want.astype(np.float32))
     assert np.isnan(y[5]).all() and np.isnan(y[6]).all()
     ref[1] *= 2.0 ** 100
