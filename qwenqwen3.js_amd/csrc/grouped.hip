@@ -28,13 +28,23 @@ struct GrMT {
 };
 
 // ---------------------------------------------------------------------------
-// Dispatch: one workgroup of NT threads; pair p is handled by thread p % NT.
-// Pass 1 counts pairs per expert with LDS atomics, one wave scans the counts
-// into offsets (and cuts the row tiles), pass 2 hands out slots with LDS
-// atomics.  The order of slots within an expert is therefore unspecified;
-// nothing depends on it: every slot row is computed on its own and the
-// combine reads slots through inv, so results are the same bit for bit.
+// Dispatch: 1 to DISP_MAX_WG workgroups; pair p is read by thread p % NT.
+// Pass 1 counts all pairs per expert with LDS atomics (every workgroup for
+// itself, those ahead of its own share apart), one wave scans the counts into
+// offsets (workgroup 0 also writes them and cuts the row tiles), and pass 2
+// hands out the slots of the workgroup's share with LDS atomics.  The order of
+// slots within an expert is therefore unspecified; nothing depends on it:
+// every slot row is computed on its own and the combine reads slots through
+// inv, so results are the same bit for bit.
+//
+// What takes the time with many pairs is pass 2's scattered stores, 64
+// different lines an instruction through one CU: hence the shares.  One
+// workgroup / shares: 16384 pairs 12.2 / 8.3 us, 8192 8.9 / 6.9, 5600 (128
+// experts) 8.4 / 6.3, 2400 6.5 / 6.1; with 8 shares of at least 2048 pairs 8.7,
+// 7.2, 7.3, 7.0.
 // ---------------------------------------------------------------------------
+constexpr int DISP_MAX_WG = 16;
+constexpr int DISP_SHARE = 512;   // pairs per workgroup, at least
 constexpr int DISP_THREADS = 1024;
 constexpr int DISP_ROUND = 16;   // pair loads in flight per thread
 
@@ -43,8 +53,11 @@ __global__ __launch_bounds__(DISP_THREADS) void moe_dispatch_kernel(
     int32_t *__restrict__ offsets, int32_t *__restrict__ perm, int32_t *__restrict__ inv,
     DispatchTiles tiles)
 {
-    __shared__ int cnt[MAX_E], cur[MAX_E], offs[MAX_E + 1];
+    __shared__ int cnt[MAX_E], cur[MAX_E], offs[MAX_E];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
+    // this workgroup's share of the pairs
+    const int share = (P + (int)gridDim.x - 1) / (int)gridDim.x;
+    const int p0 = (int)blockIdx.x * share, p1 = min(P, p0 + share);
     for (int e = tid; e < E; e += DISP_THREADS) {
         cnt[e] = 0;
         cur[e] = 0;
@@ -61,7 +74,8 @@ __global__ __launch_bounds__(DISP_THREADS) void moe_dispatch_kernel(
 #pragma unroll
         for (int i = 0; i < DISP_ROUND; i++) {
             const int e = ev[i];
-            if ((unsigned)e < (unsigned)E && !mask_has(mask, e)) atomicAdd(&cnt[e], 1);
+            if ((unsigned)e < (unsigned)E && !mask_has(mask, e))
+                atomicAdd(b0 + tid + DISP_THREADS * i < p0 ? &cur[e] : &cnt[e], 1);
         }
     }
     __syncthreads();
@@ -72,16 +86,18 @@ __global__ __launch_bounds__(DISP_THREADS) void moe_dispatch_kernel(
         int run = 0, trun = 0;
         for (int e0 = 0; e0 < E; e0 += WAVE) {
             const int e = e0 + lane;
-            const int c = e < E ? cnt[e] : 0;
+            const int c = e < E ? cur[e] + cnt[e] : 0;
             int tot;
             const int o = run + wave_excl_scan(c, &tot);
             if (e < E) {
                 offs[e] = o;
-                counts[e] = c;
-                offsets[e] = o;
+                if (blockIdx.x == 0) {
+                    counts[e] = c;
+                    offsets[e] = o;
+                }
             }
             run += tot;
-            if (tiles.bm > 0) {
+            if (blockIdx.x == 0 && tiles.bm > 0) {
                 const int nte = (c + tiles.bm - 1) / tiles.bm;
                 int ttot;
                 int t = trun + wave_excl_scan(nte, &ttot);
@@ -92,8 +108,7 @@ __global__ __launch_bounds__(DISP_THREADS) void moe_dispatch_kernel(
                 trun += ttot;
             }
         }
-        if (lane == 0) {
-            offs[E] = run;
+        if (blockIdx.x == 0 && lane == 0) {
             offsets[E] = run;
             if (tiles.bm > 0) *tiles.n = min(trun, tiles.cap);
         }
@@ -111,7 +126,8 @@ __global__ __launch_bounds__(DISP_THREADS) void moe_dispatch_kernel(
 #pragma unroll
         for (int i = 0; i < DISP_ROUND; i++) {
             const int p = b0 + tid + DISP_THREADS * i;
-            if (p >= P) break;
+            if (p >= p1) break;
+            if (p < p0) continue;
             const int e = ev[i];
             const int pos = ((unsigned)e < (unsigned)E && !mask_has(mask, e)) ? offs[e] + atomicAdd(&cur[e], 1) : -1;
             if ((unsigned)pos < (unsigned)P) {   // (always, for a routed pair)
@@ -370,7 +386,8 @@ int launch_dispatch(qq_ctx *ctx, const qq_moe *m, const int32_t *idx, int P, con
                     const DispatchTiles &tiles)
 {
     prof_begin(ctx, K_DISPATCH);
-    QQ_LAUNCH(ctx, moe_dispatch_kernel, dim3(1), dim3(DISP_THREADS), 0, idx, P, m->E, mask, counts,
+    const unsigned wgs = (unsigned)std::min(std::max(P / DISP_SHARE, 1), DISP_MAX_WG);
+    QQ_LAUNCH(ctx, moe_dispatch_kernel, dim3(wgs), dim3(DISP_THREADS), 0, idx, P, m->E, mask, counts,
               offsets, perm, inv, tiles);
     prof_end(ctx);
     QQ_HIP(ctx, hipGetLastError());
