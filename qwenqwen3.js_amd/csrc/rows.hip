@@ -7,8 +7,12 @@
 // 8 significand bits, cut off rather than rounded), and an int8 weight is a
 // bf16 value, so per 32-value block three MFMAs per k step give
 // sum(x_lo q) + sum(x_mid q) + sum(x_hi q) from exact products with fp32
-// accumulation; the block's fp16 scale is applied to that fp32 sum.  No range
-// is lost (bf16 has the exponents of fp32), so any finite row is accepted.
+// accumulation; the block's fp16 scale is applied to that fp32 sum.  bf16 has
+// the exponents of fp32 but not its 24 bits below 2^-110, and 32 unscaled
+// products of values from 2^115 on can leave fp32: a wave (GEMM: workgroup)
+// that met activations all below 2^-63, or whose sums are not finite, forms
+// its sums again from rows scaled by a power of two (scale_of).  So a finite
+// row of any magnitude, subnormals too, is taken as exactly as any other.
 // Long sums are kept in two levels (RG_FLUSH blocks, then the total).
 // Relative L2 against binary64 at 2048 -> 7168, 200 rows: 8.6e-8 (the fp32
 // vector-unit kernel this replaces: 2.2e-7).
@@ -22,6 +26,8 @@
 //     64       64.7 / 17.5    66.6 / 19.4    17.4 / 7.0      654 / 61.0
 //    200        193 / 32.7     248 / 34.8    44.2 / 16.7      -
 //   1000        950 / 105     1055 / 114      232 / 35.5      -
+#include <type_traits>
+
 #include "qq_device.h"
 
 namespace qq {
@@ -36,34 +42,68 @@ __device__ __forceinline__ uint32_t top16(uint32_t hi, uint32_t lo)
     return __builtin_amdgcn_perm(hi, lo, 0x07060302u);
 }
 
-// 8 fp32 values -> three bf16 planes with v = h + m + l exactly.  Infinities
-// go to h alone and NaN stays NaN (the differences that would turn an
-// infinity into NaN are repaired on a path no finite row takes).
+// 8 fp32 values -> three bf16 planes with v = h + m + l: exactly from 2^-110
+// on; of smaller values the bits below 2^-133 are cut off.  A NaN stays one;
+// an infinity turns into one unless INF, where it goes to h alone (on a path no
+// finite row takes).
+template <bool INF>
 __device__ __forceinline__ void split3(const float (&v)[8], uint4 &h, uint4 &m, uint4 &l)
 {
     uint32_t u[8], rb[8], lb[8];
-    float chk = 0.0f;
+    float t[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         u[i] = __float_as_uint(v[i]);
         const float r = v[i] - __uint_as_float(u[i] & 0xffff0000u);
         rb[i] = __float_as_uint(r);
-        const float t = r - __uint_as_float(rb[i] & 0xffff0000u);
-        lb[i] = __float_as_uint(t);
-        chk += t;
+        t[i] = r - __uint_as_float(rb[i] & 0xffff0000u);
+        lb[i] = __float_as_uint(t[i]);
     }
-    if (chk != chk) {
+    if constexpr (INF) {
+        float chk = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            if ((u[i] & 0x7f800000u) == 0x7f800000u) {
-                if (u[i] & 0x007fffffu) u[i] = 0x7fc00000u;
-                rb[i] = lb[i] = 0;
-            }
+        for (int i = 0; i < 8; i += 2) chk = fmaf(t[i], t[i + 1], chk);
+        if (chk != chk) {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if ((u[i] & 0x7f800000u) == 0x7f800000u) {
+                    if (u[i] & 0x007fffffu) u[i] = 0x7fc00000u;
+                    rb[i] = lb[i] = 0;
+                }
+        }
     }
     h = make_uint4(top16(u[1], u[0]), top16(u[3], u[2]), top16(u[5], u[4]), top16(u[7], u[6]));
     m = make_uint4(top16(rb[1], rb[0]), top16(rb[3], rb[2]), top16(rb[5], rb[4]), top16(rb[7], rb[6]));
     l = make_uint4(top16(lb[1], lb[0]), top16(lb[3], lb[2]), top16(lb[5], lb[4]), top16(lb[7], lb[6]));
 }
+
+// or8 collects the bits of all activations met; tiny_bits: all below 2^-63
+// (both top exponent bits clear) and not all 0.
+__device__ __forceinline__ uint32_t or8(const float (&v)[8], uint32_t o)
+{
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) o = o | __float_as_uint(v[i]) | __float_as_uint(v[i + 1]);
+    return o;
+}
+
+__device__ __forceinline__ bool tiny_bits(uint32_t o) { return (o & 0x7fffffffu) != 0 && (o & 0x60000000u) == 0; }
+
+// The same from the h planes alone, at half the instructions: a bf16 of 0 may
+// be that of a 0 or of a value below 2^-133, so the values are looked at again.
+__device__ __forceinline__ uint32_t or4(const uint4 h, uint32_t o) { return (o | h.x | h.y) | h.z | h.w; }
+__device__ __forceinline__ bool maybe_tiny(uint32_t o) { return (o & 0x60006000u) == 0; }
+
+__device__ __forceinline__ float max8(const float (&v)[8], float m)
+{
+#pragma unroll
+    for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(v[i]));
+    return m;
+}
+
+__device__ __forceinline__ bool tiny(float m) { return m > 0.0f && m < 0x1p-63f; }
+
+// The power of two that a row enters with whose largest value is m.
+__device__ __forceinline__ float scale_of(float m) { return tiny(m) ? 0x1p64f : m > 0x1p115f ? 0x1p-32f : 1.0f; }
 
 __device__ __forceinline__ b8_t as_b8(const uint4 v) { return __builtin_bit_cast(b8_t, v); }
 
@@ -177,12 +217,15 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
 #pragma unroll
         for (int m = 0; m < MF; m++) load8<RAG>(xr[m], kb, kb * QK + kq, a.in_dim, b.a[m]);
     };
-    auto mul = [&](const Blk &b) {
+    uint32_t bits[MF];
+#pragma unroll
+    for (int m = 0; m < MF; m++) bits[m] = 0;
+    auto mul_any = [&](const Blk &b, auto any) {
         b8_t ah[MF], am[MF], al[MF];
 #pragma unroll
         for (int m = 0; m < MF; m++) {
             uint4 h, mm, l;
-            split3(b.a[m], h, mm, l);
+            split3<decltype(any)::value>(b.a[m], h, mm, l);
             ah[m] = as_b8(h);
             am[m] = as_b8(mm);
             al[m] = as_b8(l);
@@ -200,6 +243,11 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
                 for (int r = 0; r < 4; r++) acc[m][f][r] = fmaf(p[r], d, acc[m][f][r]);
             }
         }
+    };
+    auto mul = [&](const Blk &b) {
+#pragma unroll
+        for (int m = 0; m < MF; m++) bits[m] = or8(b.a[m], bits[m]);
+        mul_any(b, std::false_type());
     };
 
     const int n = (a.nb - wave + RS_NW - 1) / RS_NW;   // this wave's blocks
@@ -229,6 +277,55 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
 #pragma unroll
     for (int u = 0; u < RS_PF; u++)
         if (i + u + RS_PF < n) mul(blk[u]);
+
+    // rows outside the range of the split, or sums outside that of fp32
+    float chk = 0.0f;
+    bool again = false;
+#pragma unroll
+    for (int m = 0; m < MF; m++) {
+        again = again || tiny_bits(bits[m]);
+#pragma unroll
+        for (int f = 0; f < NF; f++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) chk = fmaf(acc[m][f][r], 0.0f, chk);
+    }
+    if (__any(again || chk != 0.0f)) {   // (chk is NaN then)
+        float sc[MF];
+#pragma unroll
+        for (int m = 0; m < MF; m++) sc[m] = 0.0f;
+#pragma unroll 1
+        for (int kb = wave; kb < a.nb; kb += RS_NW) {
+            Blk b;
+            load(b, kb);
+#pragma unroll
+            for (int m = 0; m < MF; m++) sc[m] = max8(b.a[m], sc[m]);
+        }
+#pragma unroll
+        for (int m = 0; m < MF; m++) {   // lanes l, l + 16, l + 32, l + 48 hold a row
+            sc[m] = fmaxf(sc[m], __shfl_xor(sc[m], 16, WAVE));
+            sc[m] = scale_of(fmaxf(sc[m], __shfl_xor(sc[m], 32, WAVE)));
+#pragma unroll
+            for (int f = 0; f < NF; f++) acc[m][f] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll 1
+        for (int kb = wave; kb < a.nb; kb += RS_NW) {
+            Blk b;
+            load(b, kb);
+#pragma unroll
+            for (int m = 0; m < MF; m++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) b.a[m][j] *= sc[m];
+            mul_any(b, std::true_type());
+        }
+#pragma unroll
+        for (int m = 0; m < MF; m++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float inv = 1.0f / __shfl(sc[m], 4 * (lane >> 4) + r, WAVE);
+#pragma unroll
+                for (int f = 0; f < NF; f++) acc[m][f][r] *= inv;
+            }
+    }
 #pragma unroll
     for (int m = 0; m < MF; m++) {
         __syncthreads();
@@ -287,6 +384,8 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
     constexpr int NJ = NWN / 4;     // blocks of a step per wave
     static_assert(NWN == 4 || NWN == 8, "8 waves");
     __shared__ __align__(16) char lds[2 * RG_BUF];
+    __shared__ uint32_t rowmax[RG_BM];
+    __shared__ int sh_again;
     // blocks x, x+8, ... run on one XCD: each takes a contiguous run of the
     // items (row tiles of a column group and segment next to each other), so
     // the weights of a column group are read through one L2
@@ -315,9 +414,11 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
         const int kb = min(2 * (s0 + s) + ab, a.nb - 1);
         load8<RAG>(xs, kb, kb * QK + 8 * ac, a.in_dim, v);
     };
+    uint32_t bits = 0;
     auto store_a = [&](const float (&v)[8], int s, int buf) {
         uint4 h, m, l;
-        split3(v, h, m, l);
+        split3<true>(v, h, m, l);
+        bits = or4(h, bits);
         if (2 * (s0 + s) + ab >= a.nb) h = m = l = make_uint4(0, 0, 0, 0);
         char *p = xd + buf * RG_BUF;
         *reinterpret_cast<uint4 *>(p) = h;
@@ -379,6 +480,8 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
     };
     // As in the row kernel, the steady loop's loads are unconditional.
     const int last = steps - 1;
+    if (threadIdx.x < RG_BM) rowmax[threadIdx.x] = 0;
+    if (threadIdx.x == 0) sh_again = 0;
     load_a(av[0], 0);
 #pragma unroll
     for (int u = 0; u < RG_BD; u++) load_b(bs[u], min(u, last));
@@ -419,6 +522,54 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int r = 0; r < 16; r++) tot[i][r] += acc[i][r];
+    // rows outside the range of the split, or sums outside that of fp32
+    float chk = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) chk = fmaf(tot[i][r], 0.0f, chk);
+    float mx = 0.0f;
+    if (maybe_tiny(bits))
+#pragma unroll 8
+        for (int s = 0; s < steps; s++) {
+            load_a(av[0], s);
+            mx = max8(av[0], mx);
+        }
+    if (tiny(mx) || chk != 0.0f) sh_again = 1;   // (chk is NaN then)
+    __syncthreads();
+    if (sh_again) {
+#pragma unroll 4
+        for (int s = 0; s < steps; s++) {
+            load_a(av[0], s);
+            mx = max8(av[0], mx);
+        }
+        atomicMax(&rowmax[ar], __float_as_uint(mx));
+        __syncthreads();
+        const float sc = scale_of(__uint_as_float(rowmax[ar]));
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][r] = tot[i][r] = 0.0f;
+#pragma unroll 1
+        for (int s = 0; s < steps; s++) {
+            load_a(av[0], s);
+            load_b(bs[0], s);
+#pragma unroll
+            for (int j = 0; j < 8; j++) av[0][j] *= sc;
+            store_a(av[0], s, 0);
+            __syncthreads();
+            mul(bs[0], s, 0);
+            if ((s & (RG_FLUSH - 1)) == RG_FLUSH - 1) flush();
+            __syncthreads();
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int row = 32 * i + 8 * (r >> 2) + 4 * hf + (r & 3);
+                tot[i][r] = (tot[i][r] + acc[i][r]) * (1.0f / scale_of(__uint_as_float(rowmax[row])));
+            }
+    }
     if (NJ == 1) {   // the second blocks' sums pass through LDS to the waves of the first
         float *red = reinterpret_cast<float *>(lds) + wn * 2 * 16 * WAVE + lane;
         if (kg == 1) {

@@ -89,6 +89,39 @@ def test_rows_special_values(in_dim, rows):
         assert rel_l2(y[r], ref[r]) < TOL, r
 
 
+@pytest.mark.parametrize("in_dim,out_dim,rows", [
+    (512, 96, 16), (2048, 300, 24),         # row kernel: one and two row fragments
+    (2048, 4200, 12), (64, 33000, 12), (64, 8200, 24),      # ... two and four column fragments
+    (2048, 96, 100), (512, 16500, 200),     # GEMM: steps split over workgroups, 256-output groups
+    (1000, 300, 24), (1000, 300, 120),      # in_dim % 32 != 0
+])
+def test_rows_range(in_dim, out_dim, rows):
+    """Rows of every magnitude that fp32 holds, subnormals included, up to
+    where 32 unscaled products would leave it; rows beside them keep the bits
+    they have without them.  A result below 2^-126 is rounded at 2^-149 once per
+    wave and segment: at most 16 such roundings."""
+    rng = np.random.default_rng([in_dim, out_dim, rows, 9])
+    w = synth.q8_0_tensor(rng, in_dim, out_dim)
+    x = rng.standard_normal((rows, in_dim)).astype(np.float32)
+    ctx = gpu_context()
+    t = ctx.upload_q8_0(w, in_dim, out_dim)
+    try:
+        plain = t.matvec(x)
+        exps = [-145, -135, -126, -120, -112, -100, -70, -62, 112, 116, 119]
+        for r, e in enumerate(exps):
+            x[r] = (x[r].astype(np.float64) * 2.0 ** e).astype(np.float32)
+        y = t.matvec(x)
+    finally:
+        t.release()
+    ref = x.astype(np.float64) @ _dense(w, in_dim, out_dim).T
+    assert np.abs(ref).max() < 2.0 ** 127
+    for r, e in enumerate(exps):
+        err = np.linalg.norm(y[r].astype(np.float64) - ref[r])
+        bound = TOL * np.linalg.norm(ref[r]) + 16 * 2.0 ** -149 * np.sqrt(out_dim)
+        assert err < bound, (e, err / np.linalg.norm(ref[r]))
+    np.testing.assert_array_equal(y[len(exps):], plain[len(exps):])
+
+
 def test_rows_captured():
     """A recorded call needs nothing the context did not already hold, and
     replays to the eager result."""
