@@ -88,10 +88,8 @@ __device__ __forceinline__ uint32_t or8(const float (&v)[8], uint32_t o)
 
 __device__ __forceinline__ bool tiny_bits(uint32_t o) { return (o & 0x7fffffffu) != 0 && (o & 0x60000000u) == 0; }
 
-// The same from the h planes alone, at half the instructions: a bf16 of 0 may
-// be that of a 0 or of a value below 2^-133, so the values are looked at again.
-__device__ __forceinline__ uint32_t or4(const uint4 h, uint32_t o) { return (o | h.x | h.y) | h.z | h.w; }
-__device__ __forceinline__ bool maybe_tiny(uint32_t o) { return (o & 0x60006000u) == 0; }
+// Whether 8 values are all below 2^-63, from their h plane.
+__device__ __forceinline__ bool small8(const uint4 h) { return (((h.x | h.y | h.z) | h.w) & 0x60006000u) == 0; }
 
 __device__ __forceinline__ float max8(const float (&v)[8], float m)
 {
@@ -102,8 +100,12 @@ __device__ __forceinline__ float max8(const float (&v)[8], float m)
 
 __device__ __forceinline__ bool tiny(float m) { return m > 0.0f && m < 0x1p-63f; }
 
-// The power of two that a row enters with whose largest value is m.
+// The power of two that a row enters with whose largest value (NaN apart) is m.
 __device__ __forceinline__ float scale_of(float m) { return tiny(m) ? 0x1p64f : m > 0x1p115f ? 0x1p-32f : 1.0f; }
+
+// Of products of pairs of sums: finite only if all of these are (the other way
+// round only up to 2^63, past which a look at the rows does no harm).
+__device__ __forceinline__ bool finite_sum(float c) { return fabsf(c) <= 0x1.fffffep127f; }
 
 __device__ __forceinline__ b8_t as_b8(const uint4 v) { return __builtin_bit_cast(b8_t, v); }
 
@@ -278,21 +280,20 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
     for (int u = 0; u < RS_PF; u++)
         if (i + u + RS_PF < n) mul(blk[u]);
 
-    // rows outside the range of the split, or sums outside that of fp32
+    // rows outside the range of the split, or sums outside that of fp32?
     float chk = 0.0f;
-    bool again = false;
+    bool look = false, again = false;
+    float sc[MF];
 #pragma unroll
     for (int m = 0; m < MF; m++) {
-        again = again || tiny_bits(bits[m]);
+        look = look || tiny_bits(bits[m]);
+        sc[m] = 0.0f;
 #pragma unroll
         for (int f = 0; f < NF; f++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) chk = fmaf(acc[m][f][r], 0.0f, chk);
+            for (int r = 0; r < 4; r += 2) chk = fmaf(acc[m][f][r], acc[m][f][r + 1], chk);
     }
-    if (__any(again || chk != 0.0f)) {   // (chk is NaN then)
-        float sc[MF];
-#pragma unroll
-        for (int m = 0; m < MF; m++) sc[m] = 0.0f;
+    if (__any(look || !finite_sum(chk))) {
 #pragma unroll 1
         for (int kb = wave; kb < a.nb; kb += RS_NW) {
             Blk b;
@@ -304,9 +305,14 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
         for (int m = 0; m < MF; m++) {   // lanes l, l + 16, l + 32, l + 48 hold a row
             sc[m] = fmaxf(sc[m], __shfl_xor(sc[m], 16, WAVE));
             sc[m] = scale_of(fmaxf(sc[m], __shfl_xor(sc[m], 32, WAVE)));
+            again = again || sc[m] != 1.0f;
+        }
+    }
+    if (__any(again)) {
+#pragma unroll
+        for (int m = 0; m < MF; m++)
 #pragma unroll
             for (int f = 0; f < NF; f++) acc[m][f] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        }
 #pragma unroll 1
         for (int kb = wave; kb < a.nb; kb += RS_NW) {
             Blk b;
@@ -385,7 +391,7 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
     static_assert(NWN == 4 || NWN == 8, "8 waves");
     __shared__ __align__(16) char lds[2 * RG_BUF];
     __shared__ uint32_t rowmax[RG_BM];
-    __shared__ int sh_again;
+    __shared__ int sh_look;
     // blocks x, x+8, ... run on one XCD: each takes a contiguous run of the
     // items (row tiles of a column group and segment next to each other), so
     // the weights of a column group are read through one L2
@@ -414,11 +420,17 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
         const int kb = min(2 * (s0 + s) + ab, a.nb - 1);
         load8<RAG>(xs, kb, kb * QK + 8 * ac, a.in_dim, v);
     };
-    uint32_t bits = 0;
-    auto store_a = [&](const float (&v)[8], int s, int buf) {
+    uint32_t met = 0;   // chunks of small values, not all 0
+    auto store_a = [&](const float (&v)[8], int s, int buf, auto inf) {
         uint4 h, m, l;
-        split3<true>(v, h, m, l);
-        bits = or4(h, bits);
+        // (in the loop, infinities may turn into NaN: such sums are formed again.
+        // What NWN = 8 needs there is the branch: without it the compiler spills
+        // 400 bytes a lane.)
+        split3<NWN == 8 || decltype(inf)::value>(v, h, m, l);
+        if (small8(h) && (or8(v, 0) & 0x7fffffffu)) {
+            met = 1;
+            asm volatile("" : "+v"(met));   // keeps this a branch, for the same reason
+        }
         if (2 * (s0 + s) + ab >= a.nb) h = m = l = make_uint4(0, 0, 0, 0);
         char *p = xd + buf * RG_BUF;
         *reinterpret_cast<uint4 *>(p) = h;
@@ -481,12 +493,12 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
     // As in the row kernel, the steady loop's loads are unconditional.
     const int last = steps - 1;
     if (threadIdx.x < RG_BM) rowmax[threadIdx.x] = 0;
-    if (threadIdx.x == 0) sh_again = 0;
+    if (threadIdx.x == 0) sh_look = 0;
     load_a(av[0], 0);
 #pragma unroll
     for (int u = 0; u < RG_BD; u++) load_b(bs[u], min(u, last));
     load_a(av[1], min(1, last));
-    store_a(av[0], 0, 0);
+    store_a(av[0], 0, 0, std::false_type());
     load_a(av[0], min(2, last));
     __syncthreads();
     int sb = 0;
@@ -494,7 +506,7 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
 #pragma unroll
         for (int u = 0; u < RG_BD; u++) {
             const int s = sb + u;
-            store_a(av[(u + 1) & 1], s + 1, (u + 1) & 1);
+            store_a(av[(u + 1) & 1], s + 1, (u + 1) & 1, std::false_type());
             load_a(av[(u + 1) & 1], s + 3);
             __builtin_amdgcn_sched_barrier(0);
             mul(bs[u], s, u & 1);
@@ -509,7 +521,7 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
         for (int u = 0; u < RG_BD; u++) {
             const int s = sb + u;
             if (s < steps) {
-                if (s < last) store_a(av[(u + 1) & 1], s + 1, (u + 1) & 1);
+                if (s < last) store_a(av[(u + 1) & 1], s + 1, (u + 1) & 1, std::false_type());
                 if (s + 3 < steps) load_a(av[(u + 1) & 1], s + 3);
                 mul(bs[u], s, u & 1);
                 if (s + RG_BD < steps) load_b(bs[u], s + RG_BD);
@@ -522,29 +534,28 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int r = 0; r < 16; r++) tot[i][r] += acc[i][r];
-    // rows outside the range of the split, or sums outside that of fp32
+    // rows outside the range of the split, or sums outside that of fp32?
     float chk = 0.0f;
+    bool again = false;
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) chk = fmaf(tot[i][r], 0.0f, chk);
-    float mx = 0.0f;
-    if (maybe_tiny(bits))
-#pragma unroll 8
-        for (int s = 0; s < steps; s++) {
-            load_a(av[0], s);
-            mx = max8(av[0], mx);
-        }
-    if (tiny(mx) || chk != 0.0f) sh_again = 1;   // (chk is NaN then)
+        for (int r = 0; r < 16; r += 2) chk = fmaf(tot[i][r], tot[i][r + 1], chk);
+    if (met || !finite_sum(chk)) sh_look = 1;
     __syncthreads();
-    if (sh_again) {
-#pragma unroll 4
+    if (sh_look) {
+        float mx = 0.0f;
+#pragma unroll 8
         for (int s = 0; s < steps; s++) {
             load_a(av[0], s);
             mx = max8(av[0], mx);
         }
         atomicMax(&rowmax[ar], __float_as_uint(mx));
         __syncthreads();
+        // (the same in every wave: lane l looks at row l)
+        again = __any(scale_of(__uint_as_float(rowmax[lane])) != 1.0f);
+    }
+    if (again) {
         const float sc = scale_of(__uint_as_float(rowmax[ar]));
 #pragma unroll
         for (int i = 0; i < 2; i++)
@@ -556,7 +567,7 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
             load_b(bs[0], s);
 #pragma unroll
             for (int j = 0; j < 8; j++) av[0][j] *= sc;
-            store_a(av[0], s, 0);
+            store_a(av[0], s, 0, std::true_type());
             __syncthreads();
             mul(bs[0], s, 0);
             if ((s & (RG_FLUSH - 1)) == RG_FLUSH - 1) flush();
