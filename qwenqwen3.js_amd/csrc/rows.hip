@@ -124,35 +124,35 @@ __device__ __forceinline__ b8_t int8_to_bf16x8(const uint32_t w0, const uint32_t
     return __builtin_bit_cast(b8_t, make_uint4(o[0], o[1], o[2], o[3]));
 }
 
-// 8 consecutive activations of a row, k .. k + 7 of block kb (wave-uniform).
-// RAG: rows of any length and 4-byte alignment; a block that crosses the end
-// of the row is read value by value, zero from in_dim on.
+// 8 consecutive activations.  RAG: at any 4-byte alignment.
 typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
 template <bool RAG>
-__device__ __forceinline__ void load8(const float *xr, int kb, int k, int in_dim, float (&v)[8])
+__device__ __forceinline__ void load8(const float *x, float (&v)[8])
 {
-    if (RAG && kb * QK + QK > in_dim) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float t = xr[min(k + i, in_dim - 1)];
-            v[i] = k + i < in_dim ? t : 0.0f;
-        }
-        return;
-    }
     if constexpr (RAG) {
-        const f4u_t a = *reinterpret_cast<const f4u_t *>(xr + k);
-        const f4u_t b = *reinterpret_cast<const f4u_t *>(xr + k + 4);
+        const f4u_t a = *reinterpret_cast<const f4u_t *>(x);
+        const f4u_t b = *reinterpret_cast<const f4u_t *>(x + 4);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             v[i] = a[i];
             v[4 + i] = b[i];
         }
     } else {
-        const float4 a = *reinterpret_cast<const float4 *>(xr + k);
-        const float4 b = *reinterpret_cast<const float4 *>(xr + k + 4);
+        const float4 a = *reinterpret_cast<const float4 *>(x);
+        const float4 b = *reinterpret_cast<const float4 *>(x + 4);
         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
         v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    }
+}
+
+// Activations k .. k + 7 of a row of n values, zero from n on.
+__device__ __forceinline__ void load8_end(const float *xr, int k, int n, float (&v)[8])
+{
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float t = xr[min(k + i, n - 1)];
+        v[i] = k + i < n ? t : 0.0f;
     }
 }
 
@@ -209,15 +209,24 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
         for (int f = 0; f < NF; f++) acc[m][f] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     using Blk = RsBlock<MF, NF, RAG>;
-    auto load = [&](Blk &b, int kb) {
+    auto load_w = [&](Blk &b, int kb) {
         const size_t o = (size_t)kb * a.rows;
 #pragma unroll
         for (int f = 0; f < NF; f++) {
             b.q[f] = *reinterpret_cast<const uint2 *>(a.qs + (o + col[f]) * QK + kq);
             b.d[f] = a.d[o + col[f]];
         }
+    };
+    auto load = [&](Blk &b, int kb) {
+        load_w(b, kb);
 #pragma unroll
-        for (int m = 0; m < MF; m++) load8<RAG>(xr[m], kb, kb * QK + kq, a.in_dim, b.a[m]);
+        for (int m = 0; m < MF; m++) load8<RAG>(xr[m] + kb * QK + kq, b.a[m]);
+    };
+    // ... of the block that crosses the end of the row (RAG)
+    auto load_end = [&](Blk &b, int kb) {
+        load_w(b, kb);
+#pragma unroll
+        for (int m = 0; m < MF; m++) load8_end(xr[m], kb * QK + kq, a.in_dim, b.a[m]);
     };
     uint32_t bits[MF];
 #pragma unroll
@@ -252,33 +261,43 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
         mul_any(b, std::false_type());
     };
 
-    const int n = (a.nb - wave + RS_NW - 1) / RS_NW;   // this wave's blocks
-    Blk blk[RS_PF];
-    // Every load of the steady loop is unconditional: a wait for one block
-    // can then leave the blocks behind it in flight (past a branch that may
-    // or may not have issued loads the compiler has to wait for all of them).
+    // The blocks whose 32 activations all exist, then (RAG) the one that
+    // crosses the end of the row: no load of the loop is under a condition.
+    const int nfull = RAG ? a.in_dim / QK : a.nb;
+    if (!RAG || nfull > 0) {
+        const int n = (nfull - wave + RS_NW - 1) / RS_NW;   // this wave's blocks
+        Blk blk[RS_PF];
+        // Every load of the steady loop is unconditional: a wait for one block
+        // can then leave the blocks behind it in flight (past a branch that may
+        // or may not have issued loads the compiler has to wait for all of them).
 #pragma unroll
-    for (int u = 0; u < RS_PF; u++) load(blk[u], min(wave + RS_NW * u, a.nb - 1));
-    int i = 0;
-    for (; i + 2 * RS_PF <= n; i += RS_PF) {
+        for (int u = 0; u < RS_PF; u++) load(blk[u], min(wave + RS_NW * u, nfull - 1));
+        int i = 0;
+        for (; i + 2 * RS_PF <= n; i += RS_PF) {
 #pragma unroll
-        for (int u = 0; u < RS_PF; u++) {
-            mul(blk[u]);
-            // the refill behind the products
-            __builtin_amdgcn_sched_barrier(0);
-            load(blk[u], wave + RS_NW * (i + u + RS_PF));
-            __builtin_amdgcn_sched_barrier(0);
+            for (int u = 0; u < RS_PF; u++) {
+                mul(blk[u]);
+                // the refill behind the products
+                __builtin_amdgcn_sched_barrier(0);
+                load(blk[u], wave + RS_NW * (i + u + RS_PF));
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
+#pragma unroll
+        for (int u = 0; u < RS_PF; u++)
+            if (i + u < n) {
+                mul(blk[u]);
+                if (i + u + RS_PF < n) load(blk[u], wave + RS_NW * (i + u + RS_PF));
+            }
+#pragma unroll
+        for (int u = 0; u < RS_PF; u++)
+            if (i + u + RS_PF < n) mul(blk[u]);
     }
-#pragma unroll
-    for (int u = 0; u < RS_PF; u++)
-        if (i + u < n) {
-            mul(blk[u]);
-            if (i + u + RS_PF < n) load(blk[u], wave + RS_NW * (i + u + RS_PF));
-        }
-#pragma unroll
-    for (int u = 0; u < RS_PF; u++)
-        if (i + u + RS_PF < n) mul(blk[u]);
+    if (RAG && nfull < a.nb && nfull % RS_NW == wave) {
+        Blk b;
+        load_end(b, nfull);
+        mul(b);
+    }
 
     // rows outside the range of the split, or sums outside that of fp32?
     float chk = 0.0f;
@@ -297,7 +316,10 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
 #pragma unroll 1
         for (int kb = wave; kb < a.nb; kb += RS_NW) {
             Blk b;
-            load(b, kb);
+            if (RAG && kb == nfull)
+                load_end(b, kb);
+            else
+                load(b, kb);
 #pragma unroll
             for (int m = 0; m < MF; m++) sc[m] = max8(b.a[m], sc[m]);
         }
@@ -316,7 +338,10 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
 #pragma unroll 1
         for (int kb = wave; kb < a.nb; kb += RS_NW) {
             Blk b;
-            load(b, kb);
+            if (RAG && kb == nfull)
+                load_end(b, kb);
+            else
+                load(b, kb);
 #pragma unroll
             for (int m = 0; m < MF; m++)
 #pragma unroll
@@ -418,7 +443,10 @@ __global__ __launch_bounds__(RG_NT, 2) void q8_0_gemm_kernel(RowsArgs a, int nrt
     float av[2][8];
     auto load_a = [&](float (&v)[8], int s) {   // s: step from s0 on
         const int kb = min(2 * (s0 + s) + ab, a.nb - 1);
-        load8<RAG>(xs, kb, kb * QK + 8 * ac, a.in_dim, v);
+        if (RAG && kb * QK + QK > a.in_dim)   // the block that crosses the end of the row (kb is wave-uniform)
+            load8_end(xs, kb * QK + 8 * ac, a.in_dim, v);
+        else
+            load8<RAG>(xs + kb * QK + 8 * ac, v);
     };
     uint32_t met = 0;   // chunks of small values, not all 0
     auto store_a = [&](const float (&v)[8], int s, int buf, auto inf) {

@@ -66,3 +66,25 @@ def test_null_context_is_rejected():
     assert lib.qq_synchronize(None) == -1
     assert lib.qq_timer_start(None) == -1
     assert lib.qq_moe_forward(None, None, None, None, 1, None, None, None, None) == -1
+
+
+def test_code_objects_load_in_either_xnack_mode():
+    """Every kernel is built for plain gfx950: a device with XNACK on takes them too."""
+    lib = open(qq_hip.LIB_PATH, "rb").read()
+    targets = set(re.findall(rb"amdgcn-amd-amdhsa-[-a-z]*(gfx[0-9a-z:+-]+)", lib))
+    assert targets == {b"gfx950"}, targets
+
+
+def test_build_verifies_machine_code():
+    """Every kernel source (but one, for its spills of undefined values) is
+    compiled with the machine verifier on."""
+    import subprocess
+    pkg = os.path.join(ROOT, "qwenqwen3.js_amd")
+    lines = subprocess.run(["make", "-n", "-B", "-C", pkg, "ARCH=gfx950"], capture_output=True, text=True,
+                           check=True).stdout.splitlines()
+    hip = [l for l in lines if " -c " in l and l.rstrip().endswith(".hip")]
+    assert len(hip) >= 10
+    for l in hip:
+        if l.endswith("/decode.hip"):
+            continue
+        assert "-mllvm -verify-machineinstrs" in l and "--offload-arch=gfx950 " in l, l

@@ -61,6 +61,40 @@ def test_rows(in_dim, out_dim, rows):
     assert rel_l2(y, ref) < TOL
 
 
+# in_dim not a multiple of 32, or rows off alignment, through every row kernel and GEMM that 256 CUs
+# select: rows shorter than a block, of one block and a part, of a steady loop
+# and a part.  x starts 0 or 4 bytes past a 16-byte boundary, between NaN that
+# no sum may see.
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("in_dim", [20, 40, 1100, 1120])
+@pytest.mark.parametrize("out_dim,rows", [
+    (300, 1), (16500, 1),                               # a single row, aligned or not
+    (300, 5), (4100, 5), (33000, 3),                    # row kernel, 16 rows: 1, 2, 4 fragments
+    (300, 20), (2100, 20), (8200, 20),                  # ... 32 rows: 1, 2, 4 fragments
+    (300, 120), (16500, 200),                           # GEMM: 128- and 256-output groups
+])
+def test_rows_ragged(in_dim, out_dim, rows, off):
+    import torch
+    print("ragged", in_dim, out_dim, rows, off, flush=True)
+    w, x, ref = _case(in_dim, out_dim, rows, 3)
+    buf = torch.full((rows * in_dim + 8,), float("nan"), device="cuda")
+    xd = buf[off:off + rows * in_dim]
+    xd.copy_(torch.from_numpy(x).reshape(-1))
+    y = torch.full((rows, out_dim), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    ctx = gpu_context()
+    t = ctx.upload_q8_0(w, in_dim, out_dim)
+    try:
+        t.matvec_dev(xd.data_ptr(), y.data_ptr(), rows)
+        ctx.synchronize()
+    finally:
+        t.release()
+    y = y.cpu().numpy()
+    assert np.isfinite(y).all()
+    for r in range(rows):
+        assert rel_l2(y[r], ref[r]) < TOL, (r, rel_l2(y[r], ref[r]))
+
+
 @pytest.mark.parametrize("in_dim,rows", [(512, 8), (512, 24), (2048, 80), (1000, 80)])
 def test_rows_special_values(in_dim, rows):
     """Infinities, NaN and large or small rows stay with their own row; a
