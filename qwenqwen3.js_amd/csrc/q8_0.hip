@@ -67,7 +67,6 @@ int launch_repack_q8_0(qq_ctx *ctx, const uint8_t *gguf_dev, qq_tensor *t)
 // wave order.  RAG: in_dim is not a multiple of 32 (the missing activations
 // of the last block read as zero).
 constexpr int MV1_MAX_NB = 384;   // 48 KiB of activations in LDS
-constexpr int MV1_MAX_OUT = 16384;
 
 template <int RPW, int NWV, int NBW, bool RAG>
 __global__ __launch_bounds__(NWV * WAVE) void q8_0_matvec1_kernel(const int8_t *__restrict__ qs,
@@ -179,15 +178,25 @@ static void launch_matvec1(qq_ctx *ctx, const qq_tensor *t, int mat, const float
                   t->out_dim, t->nb, t->nbp, t->in_dim, x, y);
 }
 
+// Matrices whose one-row product the row kernel forms sooner: this kernel
+// stages the row once per 8 outputs, which takes long for many blocks; for very
+// few a workgroup has next to nothing else to do.  us, this kernel / the row
+// kernel: 2048 inputs, 7168 outputs 5.9 / 6.1, 16384 11.2 / 8.9, 65536 34 / 24;
+// 896 inputs, 16384 outputs 5.7 / 5.0; 768 inputs 4.3 / 4.7, 131072 outputs 23.5 /
+// 25.8; 512 inputs, 32768 outputs 4.5 / 5.1; 128 inputs 4.2 / 3.8, 50000 outputs
+// 5.6 / 5.8, 65536 6.7 / 5.9.
+static bool matvec1_large(int out_dim, int nb)
+{
+    return (nb >= 28 && out_dim >= 16384) || (nb <= 4 && out_dim >= 65536);
+}
+
 int launch_q8_0_matvec(qq_ctx *ctx, const qq_tensor *t, int mat, const float *x, int ldx,
                        float *y, int ldy, int rows)
 {
     if (rows <= 0) return QQ_OK;
-    // one vector whose activations fit in LDS (in_dim <= 12288), of a matrix of
-    // few enough outputs that staging them once per 8 outputs is cheap (us,
-    // this kernel / the row kernel, 2048 inputs: 7168 outputs 5.9 / 6.1, 16384
-    // 11.6 / 9.4, 65536 34.4 / 24.1); everything else takes the row kernels
-    if (rows > 1 || ((uintptr_t)x & 15) != 0 || t->nb > MV1_MAX_NB || t->out_dim >= MV1_MAX_OUT)
+    // one vector whose activations fit in LDS (in_dim <= 12288), of a matrix that
+    // is not large; everything else takes the row kernels
+    if (rows > 1 || ((uintptr_t)x & 15) != 0 || t->nb > MV1_MAX_NB || matvec1_large(t->out_dim, t->nb))
         return launch_q8_0_rows(ctx, t, mat, x, ldx, y, ldy, rows);
     prof_begin(ctx, K_MATVEC);
     if (t->in_dim % QK)

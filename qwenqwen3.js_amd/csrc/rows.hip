@@ -19,13 +19,13 @@
 //
 // Before, every workgroup of 32 outputs took 4 rows: the weights were read
 // and converted rows / 4 times and the products ran on the vector units.
-// us, before / now (the row kernels up to 2048 rows x blocks, else the GEMM):
-//   rows       2048 -> 7168   7168 -> 2048   1024 -> 3072   2048 -> 65536
-//      2       10.1 / 6.1     28.5 / 10.1     5.9 / 3.5     46.0 / 23.7
-//     16       21.8 / 7.3     49.5 / 16.1     8.8 / 4.2      183 / 29.8
-//     64       64.7 / 17.5    66.6 / 19.4    17.4 / 7.0      654 / 61.0
-//    200        193 / 32.7     248 / 34.8    44.2 / 16.7      -
-//   1000        950 / 105     1055 / 114      232 / 35.5      -
+// us, before / now:
+//   rows       2048 -> 7168   7168 -> 2048   1024 -> 3072   2048 -> 65536   256 -> 256
+//      2        9.6 / 5.7     28.5 / 10.4     5.9 / 3.6     39.5 / 24.1     3.7 / 3.5
+//     16       21.4 / 7.0     48.5 / 16.3     8.9 / 4.3      170 / 28.1     4.1 / 3.5
+//     64       62.1 / 13.6    65.4 / 18.9    17.9 / 6.1      629 / 58.5     4.2 / 3.6
+//    200        192 / 31.7     248 / 34.3    44.5 / 16.7      -             4.3 / 3.6
+//   1000        952 / 107     1057 / 108      232 / 35.4      -             8.9 / 4.2
 #include <type_traits>
 
 #include "qq_device.h"
@@ -712,29 +712,55 @@ int launch_q8_0_rows(qq_ctx *ctx, const qq_tensor *t, int mat, const float *x, i
         a.nvec = std::min(CHUNK, rows - v);
         const int nrt = (a.nvec + RG_BM - 1) / RG_BM;
         const int tiles = nrt * ((a.rows + 127) / 128);
-        // the row kernel reads every row once per column group: cheaper than the
-        // GEMM's steps and partial sums while rows x blocks is small (us, row
-        // kernel / GEMM: 32 rows at 2048 -> 7168 12 / 16, at 7168 -> 2048
-        // 32 / 20; 64 rows at 1024 -> 3072 7.5 / 11, at 2048 -> 7168 23 / 19)
-        if (a.nvec > 16 && (long)a.nvec * a.nb > 2048) {
+        if (a.nvec <= 16) {
+            if ((a.rows + 63) / 64 >= 2 * cu)
+                launch_rows<1, 4>(ctx, a, rag);
+            else if ((a.rows + 31) / 32 >= cu / 2)
+                launch_rows<1, 2>(ctx, a, rag);
+            else
+                launch_rows<1, 1>(ctx, a, rag);
+            continue;
+        }
+        // The row kernel in one round of the CUs, in the smallest of its tiles
+        // that makes one (2 x 2 fragments take as many workgroups as 1 x 4): its time is that of one tile, and grows with the blocks
+        // where the GEMM splits them over workgroups (us, row kernel's tiles
+        // from 16 x 16 to 32 x 64 / GEMM on a quarter of the workgroups: 8 blocks
+        // 3.9 to 5.9 / 8, 32 blocks 4.4 to 9.1 / 15, 64 blocks 6.5 to 14 / 16, 128
+        // blocks 7 to 16 / 12 to 16).
+        if (a.nb <= 64) {
+            const auto round = [&](int mf, int nf) {
+                return (long)((a.rows + 16 * nf - 1) / (16 * nf)) * ((a.nvec + 16 * mf - 1) / (16 * mf)) <= cu;
+            };
+            bool done = true;
+            if (round(1, 1))
+                launch_rows<1, 1>(ctx, a, rag);
+            else if (round(1, 2))
+                launch_rows<1, 2>(ctx, a, rag);
+            else if (round(1, 4))
+                launch_rows<1, 4>(ctx, a, rag);
+            else if (round(2, 4))
+                launch_rows<2, 4>(ctx, a, rag);
+            else
+                done = false;
+            if (done) continue;
+        }
+        // In several rounds the row kernel reads every row once per column group:
+        // cheaper than the GEMM's steps and partial sums for one row tile, or few
+        // rows x blocks (us, row kernel / GEMM: 32 rows of 7168 -> 2048 32 / 20; 24
+        // of 2048 -> 65536 47 / 55; 100 of 512 -> 8192 11.5 / 15.1, of 256 -> 8192
+        // 10.4 / 8.2, of 64 -> 8192 9.6 / 5.6)
+        if ((long)a.nvec * a.nb > 2048 || (a.nvec > 32 && a.nb < 16)) {
             // 256 outputs per workgroup where that still fills the CUs
             if (nrt * ((a.rows + 255) / 256) >= cu)
                 launch_gemm<8>(ctx, a, 1, rag);
             else   // segments of at least 4 steps; S x tiles x 32 KiB <= rows_part
                 launch_gemm<4>(ctx, a, std::max(1, std::min({cu / tiles, (a.nb + 1) / 2 / 4, RG_SMAX})), rag);
-        } else if (a.nvec > 16) {   // the widest group that leaves a quarter to half of the CUs a workgroup
-            if ((a.rows + 63) / 64 >= cu / 2)
-                launch_rows<2, 4>(ctx, a, rag);
-            else if ((a.rows + 31) / 32 >= cu / 4)
-                launch_rows<2, 2>(ctx, a, rag);
-            else
-                launch_rows<2, 1>(ctx, a, rag);
-        } else if ((a.rows + 63) / 64 >= 2 * cu) {
-            launch_rows<1, 4>(ctx, a, rag);
-        } else if ((a.rows + 31) / 32 >= cu / 2) {
-            launch_rows<1, 2>(ctx, a, rag);
+        } else if ((a.rows + 63) / 64 >= cu / 2) {   // the widest group that leaves a quarter to half of the CUs a workgroup
+            launch_rows<2, 4>(ctx, a, rag);
+        } else if ((a.rows + 31) / 32 >= cu / 4) {
+            launch_rows<2, 2>(ctx, a, rag);
         } else {
-            launch_rows<1, 1>(ctx, a, rag);
+            launch_rows<2, 1>(ctx, a, rag);
         }
     }
     prof_end(ctx);

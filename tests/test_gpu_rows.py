@@ -46,6 +46,17 @@ def _case(in_dim, out_dim, rows, seed=0):
     (1000, 1501, 4), (1000, 1501, 20), (1000, 1501, 150),   # in_dim % 32 != 0, rows 16-byte aligned
     (2048, 16383, 1), (2048, 16384, 1), (64, 40000, 1),     # one row: either side of the rule
     (1001, 77, 9), (1003, 77, 40), (33, 300, 300),          # rows at any 4-byte alignment
+    # either side of one round of the row kernel's tiles on 256 CUs: 16 x 16 outputs ...
+    (64, 2048, 32), (64, 2049, 32), (64, 4096, 32), (64, 4097, 32),
+    (512, 8192, 32), (512, 8193, 32), (64, 16384, 32), (64, 16385, 32),     # ... to 32 x 64
+    (64, 1024, 500), (64, 1024, 520),                       # many rows of few blocks, and past one round
+    (512, 8200, 33), (480, 8200, 33),                       # 16 blocks or fewer in several rounds
+    (2048, 512, 100), (2080, 512, 100),                     # 64 blocks and 65
+    (2080, 300, 20), (2080, 2100, 20), (2080, 300, 31),     # two row fragments of one and two columns
+    (96, 8300, 300), (32, 8300, 300),                       # GEMM of an odd count of blocks, of one
+    (2080, 70, 65), (4096, 31, 33),                         # GEMM: partial row and column tiles, split steps
+    (896, 16384, 1), (895, 16400, 1), (864, 16384, 1),      # one row: 28 blocks and 27,
+    (128, 65536, 1), (128, 65535, 1), (129, 65536, 1),      # 4 blocks and 5
 ])
 def test_rows(in_dim, out_dim, rows):
     print("rows", in_dim, out_dim, rows, flush=True)
@@ -66,13 +77,13 @@ def test_rows(in_dim, out_dim, rows):
 # and a part.  x starts 0 or 4 bytes past a 16-byte boundary, between NaN that
 # no sum may see.
 @pytest.mark.parametrize("off", [0, 1])
-@pytest.mark.parametrize("in_dim", [20, 40, 1100, 1120])
-@pytest.mark.parametrize("out_dim,rows", [
+@pytest.mark.parametrize("in_dim,out_dim,rows", [(i, o, r) for i in (20, 40, 1100, 1120) for o, r in (
     (300, 1), (16500, 1),                               # a single row, aligned or not
     (300, 5), (4100, 5), (33000, 3),                    # row kernel, 16 rows: 1, 2, 4 fragments
-    (300, 20), (2100, 20), (8200, 20),                  # ... 32 rows: 1, 2, 4 fragments
-    (300, 120), (16500, 200),                           # GEMM: 128- and 256-output groups
-])
+    (300, 20), (2100, 20), (4200, 20), (8200, 20),      # ... one round of tiles
+    (300, 120), (16500, 200),                           # ... GEMM of 256-output groups
+)] + [(2100, 300, 20), (2100, 2100, 20),                # 32 rows: 1 and 2 fragments
+      (2100, 300, 120), (40, 4200, 120)])               # GEMM of 128-output groups
 def test_rows_ragged(in_dim, out_dim, rows, off):
     import torch
     print("ragged", in_dim, out_dim, rows, off, flush=True)
@@ -126,8 +137,9 @@ def test_rows_special_values(in_dim, rows):
 @pytest.mark.parametrize("in_dim,out_dim,rows", [
     (512, 96, 16), (2048, 300, 24),         # row kernel: one and two row fragments
     (2048, 4200, 12), (64, 33000, 12), (64, 8200, 24),      # ... two and four column fragments
-    (2048, 96, 100), (512, 16500, 200),     # GEMM: steps split over workgroups, 256-output groups
-    (1000, 300, 24), (1000, 300, 120),      # in_dim % 32 != 0
+    (2048, 96, 100), (2048, 8200, 24),      # ... one round of tiles
+    (4096, 96, 100), (512, 16500, 200),     # GEMM: steps split over workgroups, 256-output groups
+    (1000, 300, 24), (1000, 300, 120), (2100, 300, 120),    # in_dim % 32 != 0
 ])
 def test_rows_range(in_dim, out_dim, rows):
     """Rows of every magnitude that fp32 holds, subnormals included, up to
@@ -156,12 +168,13 @@ def test_rows_range(in_dim, out_dim, rows):
     np.testing.assert_array_equal(y[len(exps):], plain[len(exps):])
 
 
-def test_rows_captured():
+@pytest.mark.parametrize("in_dim", [2048, 4096])   # row kernel; GEMM, its steps split over workgroups
+def test_rows_captured(in_dim):
     """A recorded call needs nothing the context did not already hold, and
     replays to the eager result."""
     import torch
     ctx = gpu_context()
-    in_dim, out_dim, rows = 2048, 512, 100
+    out_dim, rows = 512, 100
     w, x, _ = _case(in_dim, out_dim, rows, 2)
     t = ctx.upload_q8_0(w, in_dim, out_dim)
     xd = torch.from_numpy(x).cuda()
