@@ -104,6 +104,8 @@ def kernel_bytes(name, T, n_experts):
         return n_experts * down
     if name in ("combine", "rmsnorm"):
         return 2 * T * H * 4
+    if name == "row_inv":   # the rows read once, 8 bytes a row written
+        return T * H * 4 + T * 8
     if name == "q8_0_matvec":
         if name in LFM2_BYTES:   # the output head of the LFM2 token
             return LFM2_BYTES[name]

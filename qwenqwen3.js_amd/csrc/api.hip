@@ -123,6 +123,7 @@ static const char *const kKernelNames[K_COUNT] = {
     "dispatch",       "grouped_gateup", "grouped_down",  "combine",
     "cast_f16",         "mfma_gateup",    "mfma_down",      "stream_gateup", "stream_down",
     "rmsnorm", "lfm2_embed", "lfm2_matvec", "lfm2_attention", "route_dispatch",
+    "row_inv",
 };
 
 // After a timed-out call: clear the error word and move the epoch on by

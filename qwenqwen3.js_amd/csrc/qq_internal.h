@@ -202,6 +202,7 @@ enum KernelId {
     K_LFM2_MV,
     K_LFM2_ATTN,
     K_ROUTE_DISPATCH,
+    K_ROW_INV,
     K_COUNT
 };
 

@@ -695,7 +695,7 @@ int launch_router_topk(qq_ctx *ctx, const qq_moe *m, const float *x, int T, doub
     const int KS = ((uintptr_t)x & 15) == 0 ? router_split(m, T) : 1;
 
     if (norm) {
-        prof_begin(ctx, K_RMSNORM);
+        prof_begin(ctx, K_ROW_INV);
         QQ_LAUNCH(ctx, row_inv_kernel, dim3((T + 3) / 4), dim3(256), 0, x, T, m->H, norm->eps, norm->inv);
         prof_end(ctx);
         QQ_HIP(ctx, hipGetLastError());

@@ -60,7 +60,7 @@ def test_rmsnorm_matches_oracle(T, H):
 def test_fused_norm_moe_matches_two_calls(T, mfma, weighted, gating, H):
     """qq_moe_forward_norm_dev == qq_rmsnorm_dev then qq_moe_forward_dev, bit for bit
     (a single row is normalised inside the decode kernel, the rows of an MFMA
-    chunk inside its router launch)."""
+    chunk inside its router launch from sums of squares that a launch ahead forms)."""
     import torch
     import synth
     from _util import upload_layer
@@ -100,6 +100,32 @@ def test_fused_norm_moe_matches_two_calls(T, mfma, weighted, gating, H):
     finally:
         ctx.set_mfma_min_tokens(512)
         m.release()
+
+
+def test_fused_norm_profile_names():
+    """The launch that sums the squares ahead of the router is reported under its
+    own name: it reads the rows once, where rmsnorm's reads and writes them."""
+    import sys
+    import torch
+    import synth
+    from _util import ROOT, upload_layer
+    sys.path.insert(0, ROOT)
+    import bench
+    T, H = 600, 512
+    print("fused norm profile", T, H, flush=True)
+    ctx = gpu_context()
+    m = upload_layer(ctx, synth.moe_layer(41, H=H, F=256, E=16, K=4))
+    h = torch.randn((T, H), device="cuda")
+    torch.cuda.synchronize()
+    ctx.profile_enable(64)
+    try:
+        m.forward_norm_dev(h.data_ptr(), T, eps=1e-5)
+        prof = ctx.profile_read()
+    finally:
+        ctx.profile_enable(0)
+        m.release()
+    assert prof["row_inv"][1] == 1 and "rmsnorm" not in prof, prof
+    assert bench.kernel_bytes("row_inv", T, 16) == T * bench.H * 4 + T * 8
 
 
 def test_fused_norm_moe_decode_against_oracle():
