@@ -78,7 +78,10 @@ int qq_tensor_release(qq_ctx *ctx, qq_tensor *t);
 
 /* matmulQ80xF32 (src/tensor.js:26-53) for `rows` input vectors:
  * y[r][c] = sum_k x[r][k] * W_mat[k][c], W_mat = matrix `mat` of t.
- * x is rows*in_dim floats, y is rows*out_dim floats (host memory). */
+ * x is rows*in_dim floats, y is rows*out_dim floats (host memory).  Every row is
+ * summed in fp32 from exact products, at any magnitude; in which order depends on
+ * the shape and on how many rows a call has, so a row's last bits may differ
+ * between calls of different `rows` (never between calls of the same). */
 int qq_q8_0_matvec(qq_ctx *ctx, const qq_tensor *t, int mat, const float *x, float *y,
                    int rows);
 /* Device-pointer variant; enqueued, not waited for. */

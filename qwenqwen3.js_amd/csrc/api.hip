@@ -619,9 +619,10 @@ static size_t forward_scratch(const qq_ctx *ctx, const qq_moe *m, int T)
 
 // x, hidden (and the optional outputs) are device pointers; s holds
 // forward_scratch(ctx, m, T) bytes (256-byte aligned).  Allocates nothing.
-// With norm, x = rmsnorm(hidden) of each chunk is formed first: by the
-// router launch itself on the MFMA path (router_norm_supported), else into
-// xn (T x H floats) and x is ignored.
+// With norm, x = rmsnorm(hidden) of each chunk is formed first, and x is
+// ignored: on the MFMA path (router_norm_supported) by the router launch
+// itself, from row sums that a launch ahead writes into the chunk's part of
+// xn, else into xn (T x H floats).
 static int forward_run(qq_ctx *ctx, const qq_moe *m, const float *x, float *hidden, int T,
                        const MaskBits &mask, int32_t *idx, double *w, float *probs, char *s,
                        const NormArgs *norm = nullptr, float *xn = nullptr)
@@ -736,7 +737,7 @@ int qq_moe_forward_norm_dev(qq_ctx *ctx, const qq_moe *m, float *hidden_dev, con
         return launch_moe_decode(ctx, m, hidden_dev, hidden_dev, mb, idx_dev, w_dev, probs_dev, &norm);
     }
     // x = rmsnorm(hidden), chunk by chunk, at the start of the scratch (or
-    // formed by the router launch), then the forward
+    // formed by the router launch, the row sums there), then the forward
     const size_t xb = align256((size_t)T * m->H * 4);
     if ((rc = ensure_scratch(ctx, xb + forward_scratch(ctx, m, T)))) return rc;
     float *x = static_cast<float *>(ctx->scratch);

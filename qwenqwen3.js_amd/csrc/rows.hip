@@ -168,7 +168,8 @@ struct RowsArgs {
 
 // ---------------------------------------------------------------------------
 // A few rows (a decode batch): bound by reading the weights (2 rows of 2048 ->
-// 65536: 23.7 us, 6.0 TB/s).  A workgroup owns
+// 65536: 24 us, 5.9 TB/s; at 16 rows, 28 us, the vector units are busy half the
+// time).  A workgroup owns
 // 16 NF outputs and 16 MF input rows; its NW waves split the blocks of the
 // reduction and stream their weights (8 bytes of a column per lane and
 // fragment) straight into registers RS_PF blocks ahead, with no barrier until
@@ -382,10 +383,12 @@ __global__ __launch_bounds__(RS_NW *WAVE, 2) void q8_0_rows_kernel(RowsArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Many rows (a prompt): a GEMM on v_mfma_f32_32x32x16_bf16, bound by the
-// matrix pipe's three products per weight with the conversions beside them
-// (1000 rows of 2048 -> 7168: 280 TFLOP/s of results, 840 on the pipe; 200
-// rows: 180 and 540, one round of 224 workgroups).  Splitting the rows ahead,
+// Many rows (a prompt): a GEMM on v_mfma_f32_32x32x16_bf16 (1000 rows of 2048 ->
+// 7168: 280 TFLOP/s of results, 840 on the matrix pipe; 200 rows: 187 and 560, one
+// round of 224 workgroups).  No pipe is full at 200 rows: the vector units are
+// busy 32 % of the time with the conversions, the matrix pipes 22 % with three
+// products per weight, and the two waves of a SIMD wait a third of theirs, at a
+// barrier every step.  Splitting the rows ahead,
 // in a launch of its own, was slower (38.6 us at 200 rows against 32.7): the
 // planes are 6 bytes a value to read instead of 4.  A workgroup of 8
 // waves owns 64 input rows, 32 NWN outputs and a range of steps, a step being

@@ -17,16 +17,20 @@
 // block's fp16 scale is applied to that fp32 partial (one FMA per output),
 // as the reference applies d per block.  Error ~1e-7 relative, like the fp32
 // kernels.
-//   gate/up  A = x rows of the tile's tokens (gathered by perm), B = 64 gate +
-//            64 up columns; epilogue silu(g) * u -> act[slot][F] (fp32)
-//   down     A = act rows, B = 128 down columns -> y[slot][H] (fp32)
+//   gate/up  A = x rows of the tile's tokens (gathered by perm), B = 16 NFH gate
+//            columns and the same up columns; epilogue silu(g) * u -> act[slot][F]
+//            (fp32)
+//   down     A = act rows, B = 32 NFH down columns -> y[slot][H] (fp32)
 // followed by the gather combine.
 //
 // us per call before / now, LFM2 shape (H 2048, F 1792, 32 experts, top-4):
 // 2 tokens 47 / 38, 6 tokens 71 / 56, 12 tokens 77 / 71, 64 tokens 86 / 83,
 // 128 tokens 120 / 113; Qwen3 shape (F 768, 128 experts, top-8): 16 tokens
 // 105 / 96, 64 tokens 139 / 130.  From the steady loop's unconditional loads
-// (st_mainloop) and, up to ~12 tokens, the width of the items (st_width).
+// (st_mainloop) and, up to ~12 tokens, the width of the items (st_width).  The
+// conversion outside inline assembly (int8_to_f16x8) takes five instructions per
+// four weights instead of four, which a launch of two row fragments on few experts
+// feels: 8 experts of H 1024, F 3584, top-2, 100 tokens 62.8 / 65.5.
 #include "qq_device.h"
 
 namespace qq {
@@ -308,7 +312,8 @@ constexpr int ST_SEG_MAX = 8;   // segments of a split item
 // in flight, so with few tiles the time is that of one item, and an item's
 // time is its width (gate/up, one round: 15 us at 2, 24.8 at 4, 43.7 at 7).
 // The count of row tiles is known on the device only (the experts a few tokens
-// touch), so every workgroup works the width out; the sums do not depend on it.
+// touch), so every workgroup works the width out.  An item's own sums do not depend
+// on it; which items are left for a last round, and split (st_work), does.
 constexpr int ST_GU_MIN = 2, ST_GU_MAX = 7, ST_DN_MIN = 2, ST_DN_MAX = 4;
 
 template <int LO, int HI>
