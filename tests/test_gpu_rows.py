@@ -106,11 +106,13 @@ def test_rows_ragged(in_dim, out_dim, rows, off):
         assert rel_l2(y[r], ref[r]) < TOL, (r, rel_l2(y[r], ref[r]))
 
 
-@pytest.mark.parametrize("in_dim,rows", [(512, 8), (512, 24), (2048, 80), (1000, 80)])
-def test_rows_special_values(in_dim, rows):
+@pytest.mark.parametrize("in_dim,out_dim,rows", [
+    (512, 96, 8), (512, 96, 24), (2048, 96, 80), (1000, 96, 80),
+    (4096, 96, 80), (2100, 96, 80), (512, 16500, 200),      # GEMM: split steps, ragged, 256-output groups
+])
+def test_rows_special_values(in_dim, out_dim, rows):
     """Infinities, NaN and large or small rows stay with their own row; a
     power of two on a row is a power of two on its result."""
-    out_dim = 96
     w, x, ref = _case(in_dim, out_dim, rows, 1)
     x[1] *= np.float32(2.0 ** 100)
     x[2] *= np.float32(2.0 ** -80)
